@@ -185,39 +185,44 @@ GemmArgs gemm8(const uint8_t* A, int lda, const int* a_src, const uint8_t* as, c
   return g;
 }
 
-// K splits of the deferred GEMMs of a call of N tokens (0: no deferral): enough workgroups to occupy the 256 CUs, at
-// most 4 (the row kernels' limit), and the sums must fit the partial area; 0 unless the deferred GEMMs of the kind fit
-// the small-row kernel.  The conv GEMMs (taps) run on 64-row tiles above 32 tokens (gemm_small_part64), proj and fc2
-// on 32-row tiles (measured faster for them: K = 1024 / 2048 leaves 64-row tiles too few steps per workgroup).
-int defer_splits(const t2w_dit_dims& d, int N, const Work& w, bool taps) {
+// K splits of a deferred GEMM, [N, H] from K, whose result a row kernel finishes (splits < 2: not deferred): at most 4
+// (the row kernels' limit), and the sums must fit the partial area.  Up to 128 rows it runs on the small-row kernel
+// (ring_cfg < 0), with enough workgroups to occupy the 256 CUs: its weights come from HBM, and a workgroup that issues
+// all its loads at once waits less for them than one that keeps three ring stages in flight (in a one-window solve
+// conv 7.1 us against 7.7, proj and fc2 5.6 against 5.8).  Beyond, on the ring tiles.
+struct Defer {
+  int splits, ring_cfg;
+};
+Defer defer_plan(const t2w_dit_dims& d, int N, int K, const Work& w, bool taps) {
   const int H = d.hidden;
-  if (N > GEMM_SMALL_MAX_M || !w.part) return 0;
+  if (!w.part) return Defer{1, -1};
+  const int most = (int)std::min<size_t>(4, w.part_bytes / ((size_t)N * H * 4));
+  if (N > GEMM_SMALL_MAX_M) {
+    const RingPlan rp = ring_plan(N, H, K, std::max(most, 1), false);
+    return Defer{rp.cfg < 0 ? 1 : rp.splits, rp.cfg};
+  }
+  // the conv GEMMs (taps) run on 64-row tiles above 32 tokens (gemm_small_part64), proj and fc2 on 32-row tiles
+  // (measured faster for them: K = 1024 / 2048 leaves 64-row tiles too few steps per workgroup)
   const int rows = taps && N > 32 ? 64 : 32;
   const int tiles = ((N + rows - 1) / rows) * ((H + 31) / 32);
-  const int S = std::min(4, 256 / tiles);
-  if (S < 2 || (size_t)S * N * H * 4 > w.part_bytes) return 0;
+  const int S = std::min(most, 256 / tiles);
   static const int taps_marker = 0;  // gemm_small_fits checks only the presence of a frame id list
   GemmArgs g{};
-  g.M = N; g.N = H; g.ldc = H; g.splits = S; g.tapC = H;
-  for (int K : taps ? std::initializer_list<int>{3 * H} : std::initializer_list<int>{H, d.ffn}) {
-    g.K = K;
-    g.ldb = K;
-    g.lda = taps ? H : K;
-    g.a_src = taps ? &taps_marker : nullptr;
-    if (!gemm_small_fits(g, EPI_PART)) return 0;
-  }
-  return S;
+  g.M = N; g.N = H; g.ldc = H; g.splits = S; g.tapC = H; g.K = K; g.ldb = K;
+  g.lda = taps ? H : K;
+  g.a_src = taps ? &taps_marker : nullptr;
+  return Defer{S >= 2 && gemm_small_fits(g, EPI_PART) ? S : 1, -1};
 }
 
 // g (its bias and gate excepted) as a K-split GEMM into the partial area; the returned Pend finishes it
-Pend gemm_deferred(GemmArgs g, int S, const Work& w, hipStream_t st, hipError_t* err) {
+Pend gemm_deferred(GemmArgs g, const Defer& df, const Work& w, hipStream_t st, hipError_t* err) {
   Pend p;
-  p.part = w.part; p.S = S; p.stride = (size_t)g.M * g.N; p.ld = g.N; p.bias = g.bias; p.gate = g.gate;
+  p.part = w.part; p.S = df.splits; p.stride = (size_t)g.M * g.N; p.ld = g.N; p.bias = g.bias; p.gate = g.gate;
   g.C = w.part;
   g.ldc = g.N;
-  g.splits = S;
+  g.splits = df.splits;
   g.c_split = p.stride;
-  *err = gemm_small(g, EPI_PART, st);
+  *err = df.ring_cfg < 0 ? gemm_small(g, EPI_PART, st) : gemm_ring(g, EPI_PART, df.ring_cfg, st);
   return p;
 }
 
@@ -253,8 +258,12 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
   };
   // Calls of few tokens: the gated-residual GEMMs and conv1 split K over several workgroups per tile and the row
   // kernel that reads their result next finishes their epilogue (pend: the result it has to finish).
-  const int Sd = f8 ? 0 : defer_splits(d, N, w, false), St = f8 ? 0 : defer_splits(d, N, w, true);
-  const bool S = Sd > 0 && St > 0;  // deferral on: proj / fc2 split Sd ways, conv1 / conv2 St ways
+  Defer df_proj{1, -1}, df_conv = df_proj, df_fc2 = df_proj;
+  if (!f8) {
+    df_proj = defer_plan(d, N, H, w, false);
+    df_conv = defer_plan(d, N, 3 * H, w, true);
+    df_fc2 = defer_plan(d, N, F, w, false);
+  }
   Pend pend;
   hipError_t perr = hipSuccess;
   for (int b = 0; b < D; ++b) {
@@ -281,7 +290,13 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     }
     gq.qk = QkvOut{w.q, kp, vp, a->new_slot, k.qn_w, k.qn_b, k.kn_w, k.kn_b, d.eps_qk, H, m->g.rope_freq, a->tok_abs};
     const bool small_qkv = gemm_small_fits(gq, EPI_QKV);
-    if (small_qkv || (!gemm_splits(gq) && H % 256 == 0)) {
+    GemmArgs gr = gq;
+    gr.qk.rfreq = nullptr;
+    const RingPlan rp_qkv = f8 ? RingPlan{-1, 1} : ring_plan(N, 3 * H, H, 1, true);
+    if (!small_qkv && rp_qkv.cfg >= 0 && gemm_ring_fits(gr, EPI_QKV)) {
+      T2W_CHECK(gemm_ring(gr, EPI_QKV, rp_qkv.cfg, st), "qkv");
+      if (m->g.rope_freq) T2W_CHECK(rope_qk(w.q, kp, a->new_slot, a->tok_abs, m->g.rope_freq, N, H, st), "rope");
+    } else if (small_qkv || (!gemm_splits(gq) && H % 256 == 0)) {
       // per-head q / k LayerNorm and the key / value scatter in the projection's epilogue; the small-row kernel also
       // rotates q and k, the tile kernel leaves that to rope_qk (the sine and cosine would spill its registers)
       if (!small_qkv) gq.qk.rfreq = nullptr;
@@ -302,10 +317,10 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     T2W_CHECK(attention(at, st), "attention");
     if (f8)
       T2W_CHECK(gemm_bf16(gemm8(w.o8, H, nullptr, w.o8s, k8->proj_w8, k8->proj_ws, k.proj_b, g_a, w.h, H, N, H, H), EPI_RESID_F16, st), "proj");
-    else if (S) {
+    else if (df_proj.splits > 1) {
       const void* pw = wt(k.proj_w, k8 ? k8->proj_w8 : nullptr, k8 ? k8->proj_ws : nullptr, H, H);
       T2W_CHECK(derr, "dequant proj");
-      pend = gemm_deferred(gemm_args(w.ao, H, nullptr, pw, k.proj_b, g_a, w.h, H, N, H, H, &w), Sd, w, st, &perr);
+      pend = gemm_deferred(gemm_args(w.ao, H, nullptr, pw, k.proj_b, g_a, w.h, H, N, H, H, &w), df_proj, w, st, &perr);
       T2W_CHECK(perr, "proj");
     } else {
       const void* pw = wt(k.proj_w, k8 ? k8->proj_w8 : nullptr, k8 ? k8->proj_ws : nullptr, H, H);
@@ -327,8 +342,8 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     } else {
       const void* cw = wt(k.c1_w, k8 ? k8->c1_w8 : nullptr, k8 ? k8->c1_ws : nullptr, H, 3 * H);
       T2W_CHECK(derr, "dequant conv1");
-      if (S) {
-        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w), St, w, st, &perr);
+      if (df_conv.splits > 1) {
+        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w), df_conv, w, st, &perr);
         T2W_CHECK(perr, "conv1");
       } else {
         T2W_CHECK(gemm_bf16(gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w), EPI_BF16, st), "conv1");
@@ -344,8 +359,8 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     } else {
       const void* cw = wt(k.c2_w, k8 ? k8->c2_w8 : nullptr, k8 ? k8->c2_ws : nullptr, H, 3 * H);
       T2W_CHECK(derr, "dequant conv2");
-      if (S) {
-        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w), St, w, st, &perr);
+      if (df_conv.splits > 1) {
+        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w), df_conv, w, st, &perr);
         T2W_CHECK(perr, "conv2");
       } else {
         T2W_CHECK(gemm_bf16(gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w), EPI_RESID_F16, st), "conv2");
@@ -368,8 +383,8 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
       T2W_CHECK(gemm_bf16(gemm_args(w.abuf, H, nullptr, f1w, k.fc1_b, nullptr, w.big, F, N, F, H, &w), EPI_GELU_BF16, st), "fc1");
       const void* f2w = wt(k.fc2_w, k8 ? k8->fc2_w8 : nullptr, k8 ? k8->fc2_ws : nullptr, H, F);
       T2W_CHECK(derr, "dequant fc2");
-      if (S) {
-        pend = gemm_deferred(gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w), Sd, w, st, &perr);
+      if (df_fc2.splits > 1) {
+        pend = gemm_deferred(gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w), df_fc2, w, st, &perr);
         T2W_CHECK(perr, "fc2");
       } else {
         T2W_CHECK(timed_launch(T2W_TIMER_RESID_GEMM, resid_bytes(N, H, F), st, [&] { return gemm_bf16(gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w), EPI_RESID_F16, st); }), "fc2");

@@ -228,6 +228,10 @@ hipError_t gemm_bf16(const GemmArgs& g, int epi, hipStream_t st, int cfg) {
   if ((size_t)(g.M + 65536) * g.lda * es >= ((size_t)1 << 32) || (size_t)g.N * g.ldb * es >= ((size_t)1 << 32))
     return hipErrorInvalidValue;
   if (cfg < 0 && gemm_small_fits(g, epi)) return gemm_small(g, epi, st);
+  if (cfg < 0 && epi != EPI_PART && gemm_ring_fits(g, epi)) {
+    const RingPlan rp = ring_plan(g.M, g.N, g.K, 1, epi == EPI_QKV);
+    if (rp.cfg >= 0) return gemm_ring(g, epi, rp.cfg, st);
+  }
   // the tile epilogues store bf16 rows 16 bytes per lane
   const bool bf16_out = epi == EPI_BF16 || epi == EPI_GELU_BF16 || epi == EPI_RESID_F16 || epi == EPI_F16;  // 16-bit rows
   if (bf16_out && (g.ldc % 8 || ((size_t)g.C & 15)) && !(cfg < 0 && gemm_splits(g))) return hipErrorInvalidValue;

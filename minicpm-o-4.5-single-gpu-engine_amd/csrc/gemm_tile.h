@@ -31,7 +31,7 @@ struct Cols {
   __device__ __forceinline__ Cols(const GemmArgs& g, int n_) : n(n_), full(n_ + 3 < g.N), act(EPI == EPI_BF16 ? g.act : 0) {
     bias = gate = make_float4(0.f, 0.f, 0.f, 0.f);
     wsc = make_float4(1.f, 1.f, 1.f, 1.f);
-    if (full) {
+    if (full && EPI != EPI_PART) {  // EPI_PART: the plain sums
       bias = *(const float4*)(g.bias + n);
       if (EPI == EPI_RESID_F16) gate = *(const float4*)(g.gate + n);
       if (SC && g.w_scale) wsc = *(const float4*)(g.w_scale + n);
@@ -63,7 +63,7 @@ struct Cols {
   __device__ __forceinline__ void put_partial(const GemmArgs& g, int m, float4 a) const {
     const float v[4] = {a.x, a.y, a.z, a.w};
     for (int e = 0; e < 4 && n + e < g.N; ++e) {
-      const float x = v[e] * (SC && g.w_scale ? g.w_scale[n + e] : 1.0f) + g.bias[n + e];
+      const float x = EPI == EPI_PART ? v[e] : v[e] * (SC && g.w_scale ? g.w_scale[n + e] : 1.0f) + g.bias[n + e];
       const size_t o = (size_t)m * g.ldc + n + e;
       if (EPI == EPI_BF16) ((bf16_t*)g.C)[o] = f2bf(act_apply(x, act));
       else if (EPI == EPI_GELU_BF16) ((bf16_t*)g.C)[o] = f2bf(gelu_tanh(x));

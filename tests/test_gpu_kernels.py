@@ -173,6 +173,35 @@ def test_gemm_splitk(dev, M, N, K, epi):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 64, 64), (129, 3072, 128), (191, 72, 192), (193, 1024, 256), (321, 1024, 1024), (449, 1000, 320),
+                                   (1025, 2048, 64), (1300, 1024, 2048), (2049, 1024, 448), (4096, 1024, 128)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3, 7])
+def test_gemm_ring(dev, M, N, K, epi):
+    """The ring-buffered tiles (64x64, 128x64, 128x128 by shape) at the edges of tiles, of the ring (K of one to eight
+    stages) and of the output columns; dense and, where the epilogue has it, taps (rows of K / 64 64-value frames),
+    which read the same values and so give the same bits.  Bounds: one bf16 rounding is at most 2^-9 of a value, one
+    fp16 rounding 2^-12, fp32 sums of up to 2048 products stay within 1e-5."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K + epi)
+    F, C64 = M + K // 64 - 1, 64
+    frames = torch.randn(F, C64, device=dev, generator=g).bfloat16()  # row m: frames m .. m + K / 64 - 1
+    A = torch.cat([frames[j:j + M] for j in range(K // 64)], 1).contiguous()
+    W = (torch.randn(N, K, device=dev, generator=g) / K ** 0.5).bfloat16()
+    bias, gate = torch.randn(N, device=dev, generator=g), torch.randn(N, device=dev, generator=g)
+    h0 = torch.randn(M, N, device=dev, generator=g).half()
+    ref = A.float() @ W.float().t() + bias
+    ref = {1: torch.nn.functional.gelu(ref, approximate="tanh"), 2: h0.float() + gate * ref}.get(epi, ref)
+    outs = []
+    for taps in (False, True) if epi in (0, 2, 3) else (False,):
+        out = h0.clone() if epi == 2 else torch.full((M, N), 7.0, device=dev).to({3: torch.float32, 7: torch.float16}.get(epi, torch.bfloat16))
+        if taps:
+            _gemm(frames, W, bias, out, epi, gate=gate, a_src=torch.arange(M, dtype=torch.int32, device=dev), lda=C64, K=K)
+        else:
+            _gemm(A, W, bias, out, epi, gate=gate)
+        assert rel(out.float(), ref) < {0: 6e-3, 1: 6e-3, 2: 1e-3, 3: 1e-5, 7: 1e-3}[epi]
+        outs.append(out)
+    assert torch.equal(outs[0], outs[-1])
+
+
 def test_gemm_splitk_taps(dev):
     """Split-K in taps mode (a streaming chunk's conv GEMM) equals the tile kernel's result for the same call."""
     H, lens = 512, [50, 50]
