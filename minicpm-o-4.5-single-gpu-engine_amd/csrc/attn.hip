@@ -551,9 +551,14 @@ __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(4
 
 hipError_t attention(const AttnArgs& a, hipStream_t st) {
   if (a.n_tiles <= 0) return hipSuccess;
-  // a grid of fewer workgroups than CUs (a streaming chunk) splits each workgroup's key tiles over four wave groups
+  // a grid of fewer workgroups than CUs (a streaming chunk) splits each workgroup's key tiles over four wave groups; one
+  // of up to about two per CU (several streaming windows, prompts) over two, since their serial key tiles and not
+  // the CUs bound it: in a solve of five windows 20.6 -> 19.1 ms, of a 300-frame prompt 20.7 -> 20.3 ms (four groups
+  // there: 19.6 and 21.4 ms; two groups on sixteen windows, 992 workgroups: no change)
   if (a.n_tiles * a.heads < 256) {
     hipLaunchKernelGGL(attn_kernel<4>, dim3(a.n_tiles, a.heads), dim3(512), 0, st, a);
+  } else if (a.n_tiles * a.heads < 600) {
+    hipLaunchKernelGGL(attn_kernel<2>, dim3(a.n_tiles, a.heads), dim3(256), 0, st, a);
   } else if (a.kv_max > 0 && a.kv_max <= ATTN_ROW_KMAX && (long)a.n_rows * a.heads >= 256 && a.n_tiles >= 3 * a.n_rows) {
     // rows of three or more query tiles on average: with fewer, most of a row workgroup's waves would idle while its
     // whole key list is copied (the tile kernel is faster there)

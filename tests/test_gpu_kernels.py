@@ -347,6 +347,14 @@ def test_attention_paged_block_causal(dev, chunk, rep):
 
 
 @pytest.mark.parametrize("chunk", [0, 50])
+@pytest.mark.parametrize("rep", [8, 18, 19])
+def test_attention_key_groups(dev, chunk, rep):
+    """Grids of 256 and 576 workgroups split the key tiles over two wave groups (rows with fewer key tiles than groups
+    among them), 608 keep one."""
+    _attention_case(dev, [50, 1, 0, 130, 64, 65] * rep, [300, 0, 7, 0, 100, 33] * rep, 4, chunk, 5 + chunk + rep)
+
+
+@pytest.mark.parametrize("chunk", [0, 50])
 def test_attention_stream_chunk(dev, chunk):
     """The streaming chunk's call (a CFG pair of 50 new frames over 300 and 462 cached keys, 16 heads) with the
     planner's key bound: the bound leaves small calls on the tile kernel (the same bits) and the result matches fp32."""
