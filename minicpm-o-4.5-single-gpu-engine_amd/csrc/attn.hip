@@ -82,6 +82,24 @@ __device__ __forceinline__ void nan_rows(const AttnArgs& a, int start, int q0, i
   }
 }
 
+// Workgroup b of n reads its share of the weight ranges, four loads per thread in flight, and discards the values (an
+// empty asm keeps the loads).
+__device__ __forceinline__ void attn_prefetch(const AttnArgs& a, int b, int n) {
+  const size_t step = (size_t)n * blockDim.x;
+  uint32_t x = 0;
+  for (int r = 0; r < AttnArgs::PF_RANGES; ++r) {
+    const uint4* p = (const uint4*)a.pf[r];
+    const size_t units = a.pf_bytes[r] / 16;
+    size_t i = (size_t)b * blockDim.x + threadIdx.x;
+    for (; i + 3 * step < units; i += 4 * step) {
+      const uint4 v0 = p[i], v1 = p[i + step], v2 = p[i + 2 * step], v3 = p[i + 3 * step];
+      x ^= v0.x ^ v1.x ^ v2.x ^ v3.x;
+    }
+    for (; i < units; i += step) x ^= p[i].x;
+  }
+  asm volatile("" ::"v"(x));
+}
+
 // KS > 1 (few workgroups, e.g. a streaming chunk): KS groups of two waves share the 64 queries and take every KS-th
 // key tile each; their softmax states (max, sum, output) are merged through LDS at the end.
 template <int KS>
@@ -90,10 +108,14 @@ __global__ void __launch_bounds__(128 * KS, 2) attn_kernel(AttnArgs a) {
   __shared__ uint4 vt[KS][2][64 * 8];      // [key][16-byte chunk ^ (key & 7)], 64 keys
   // XCD-aware order: consecutive workgroups go to different XCDs, so each XCD takes a contiguous run of (head, tile)
   // pairs; the query tiles of one row and head then share that row's keys and values in one L2
-  const int nblk = gridDim.x * gridDim.y, full = (nblk / 8) * 8;
-  int lin = blockIdx.y * gridDim.x + blockIdx.x;
+  const int nblk = a.n_tiles * a.heads, full = (nblk / 8) * 8;
+  int lin = blockIdx.x;
+  if (lin >= nblk) {
+    attn_prefetch(a, lin - nblk, gridDim.x - nblk);
+    return;
+  }
   if (lin < full) lin = (lin % 8) * (nblk / 8) + lin / 8;
-  const int tile = lin % gridDim.x, head = lin / gridDim.x;
+  const int tile = lin % a.n_tiles, head = lin / a.n_tiles;
   const int gi = threadIdx.x >> 7, tid = threadIdx.x & 127, lane = tid & 63, wave = tid >> 6;
   const int row = a.tiles[2 * tile];
   const int q0 = a.tiles[2 * tile + 1];
@@ -551,14 +573,21 @@ __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(4
 
 hipError_t attention(const AttnArgs& a, hipStream_t st) {
   if (a.n_tiles <= 0) return hipSuccess;
+  const int wgs = a.n_tiles * a.heads;
+  // Prefetch workgroups: 128 of 512 threads (or as many threads in smaller ones).  In a one-window solve (28 MB of
+  // weights behind a 10 us attention) 32 left it at 15.2 ms and 256 at 14.5, their reads outlasting or delaying the
+  // attention's; 64, 128 and 192 took 13.9 ms to 13.5, 13.3 and 13.4.
+  size_t pf = 0;
+  for (int r = 0; r < AttnArgs::PF_RANGES; ++r) pf += a.pf_bytes[r];
+  const int pfw = pf ? 128 : 0;
   // a grid of fewer workgroups than CUs (a streaming chunk) splits each workgroup's key tiles over four wave groups; one
   // of up to about two per CU (several streaming windows, prompts) over two, since their serial key tiles and not
   // the CUs bound it: in a solve of five windows 20.6 -> 19.1 ms, of a 300-frame prompt 20.7 -> 20.3 ms (four groups
   // there: 19.6 and 21.4 ms; two groups on sixteen windows, 992 workgroups: no change)
-  if (a.n_tiles * a.heads < 256) {
-    hipLaunchKernelGGL(attn_kernel<4>, dim3(a.n_tiles, a.heads), dim3(512), 0, st, a);
-  } else if (a.n_tiles * a.heads < 600) {
-    hipLaunchKernelGGL(attn_kernel<2>, dim3(a.n_tiles, a.heads), dim3(256), 0, st, a);
+  if (wgs < 256) {
+    hipLaunchKernelGGL(attn_kernel<4>, dim3(wgs + pfw), dim3(512), 0, st, a);
+  } else if (wgs < 600) {
+    hipLaunchKernelGGL(attn_kernel<2>, dim3(wgs + 2 * pfw), dim3(256), 0, st, a);
   } else if (a.kv_max > 0 && a.kv_max <= ATTN_ROW_KMAX && (long)a.n_rows * a.heads >= 256 && a.n_tiles >= 3 * a.n_rows) {
     // rows of three or more query tiles on average: with fewer, most of a row workgroup's waves would idle while its
     // whole key list is copied (the tile kernel is faster there)
@@ -575,7 +604,7 @@ hipError_t attention(const AttnArgs& a, hipStream_t st) {
     else  // one workgroup of 16 waves per CU
       hipLaunchKernelGGL(attn_row_kernel<16>, dim3(a.heads, a.n_rows), dim3(64 * 16), lds, st, a);
   } else {
-    hipLaunchKernelGGL(attn_kernel<1>, dim3(a.n_tiles, a.heads), dim3(128), 0, st, a);
+    hipLaunchKernelGGL(attn_kernel<1>, dim3(wgs + 4 * pfw), dim3(128), 0, st, a);
   }
   return hipGetLastError();
 }

@@ -166,6 +166,11 @@ struct AttnArgs {
   uint8_t* out8s = nullptr;
   int n_rows = 0;            // rows of the call (the row-resident kernel's grid)
   int kv_max = 0;            // 0, or the caller's bound on every row's key-list length (for every replay of a graph)
+  // byte ranges (weights of the GEMMs that follow) that the tile kernel also reads, in workgroups of its own behind the
+  // attention's, so that they are in the memory-side cache; the values are discarded
+  static constexpr int PF_RANGES = 6;
+  const void* pf[PF_RANGES] = {};
+  size_t pf_bytes[PF_RANGES] = {};
 };
 constexpr int ATTN_ROW_KMAX = 512;  // the longest key list the row-resident attention holds in LDS
 hipError_t attention(const AttnArgs& a, hipStream_t st);
