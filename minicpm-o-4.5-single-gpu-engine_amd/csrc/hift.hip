@@ -994,130 +994,149 @@ __global__ void __launch_bounds__(256, 2) resblock_pair_kernel(ConvDesc c1, Conv
 
 // Small grids (a streaming window: one item of a few thousand samples) leave most CUs idle with whole-slab tiles, and
 // each tile's tap loop is a chain of weight-load latencies.  Here a workgroup of CS_WAVES waves owns 32 output rows x
-// NB * 32 output channels and splits the (tap, 64-channel input chunk) steps over its waves, the next step's loads
-// issued before this step's MFMAs; the waves' fp32 blocks are summed through LDS in wave order (deterministic) and the
-// epilogue writes four channels per thread.  A CU's load throughput bounds these calls, so (as in the small-row GEMM)
-// the loads cover whole lines: a step's weights are NB * 32 rows of 128 bytes, eight lanes per row; its activations 32
-// rows of 64 fp32 channels, sixteen lanes per row (activation applied, rounded to bf16).  Both go through the wave's
-// LDS slab (16-byte chunks XOR-swizzled by (row / 2) % 8) and come back as MFMA fragments.  NB = 1 halves the weight
-// bytes each workgroup reads where the grid stays within the chip.  MFMA roles as in the small-row GEMM: the weights
-// are the A operand (32 output channels), the activations the B operand (32 output rows).
+// NB * 32 output channels and splits the (tap, 64-channel input chunk) steps over its waves.  The input rows that any tap
+// reads (32 + the taps' span, all channels) are loaded once, activated once and kept in LDS as bf16; each wave's
+// weights come straight from the fragment-ordered copy (one contiguous kilobyte per fragment), the first steps' loads
+// issued before the slab is filled.  The waves' fp32 blocks are summed through LDS in wave order (deterministic) and the
+// epilogue writes four channels per thread.  MFMA roles as in the small-row GEMM: the weights are the A operand (32
+// output channels), the activations the B operand (32 output rows).
+//
+// A CU's load throughput and the Snakes bounded the kernel before this one, which loaded and activated its input rows
+// once per tap (at kernel 11, 11 x 8 KB per chunk where the slab takes 21 KB).  One launch takes up to CONV_BATCH independent convs
+// (the three ResBlocks of a stage, or the source ResBlocks of the three stages), whose grids alone leave CUs idle.
+// One 58-frame window, reference split: 1264 -> 685 us a call (88 launches -> 51).  Two workgroups share a CU
+// (128 registers): with more rows in flight per thread and one workgroup it was 16-30% slower.
 constexpr int CS_WAVES = 8;
 
+struct ConvBatch {
+  ConvDesc d[CONV_BATCH];
+  int start[CONV_BATCH + 1];  // first workgroup of each conv
+  int nx[CONV_BATCH];         // its 32-row tiles
+  int n;
+};
+
+constexpr int CW_LDS = 160 * 1024;  // a CU's LDS
+
+// slab rows in 16-byte units: a multiple of 8 that is 8 modulo 16, so that with chunks XOR-swizzled by (row / 2) % 8 the
+// fragment reads of 16 consecutive rows cover all 64 banks
+__host__ __device__ constexpr int cw_stride(int Cin) {
+  const int c = ((Cin + 63) & ~63) / 8;
+  return c % 16 ? c : c + 8;
+}
+
 template <int NB>
-__global__ void __launch_bounds__(64 * CS_WAVES) conv_bf16_split_kernel(ConvDesc c, const bf16_t* __restrict__ wbf) {
+__global__ void __launch_bounds__(64 * CS_WAVES, 4) conv_bf16_window_kernel(ConvBatch cb) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  __shared__ u32x4 slab[CS_WAVES][(NB + 1) * 256];  // per wave: W rows then activation rows of a step; then its blocks
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, cl = lane & 31;
-  const int b = blockIdx.z / c.n_phase, ph = blockIdx.z % c.n_phase;
+  extern __shared__ uint4 wlds[];  // the input slab, then the waves' blocks
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, cl = lane & 31;
+  int which = 0;
+#pragma unroll
+  for (int i = 1; i < CONV_BATCH; ++i) which += i < cb.n && (int)blockIdx.x >= cb.start[i];
+  const ConvDesc& c = cb.d[which];
+  int lb = blockIdx.x - cb.start[which];
+  const int nx = cb.nx[which], ny = (c.Cout + NB * 32 - 1) / (NB * 32);
+  const int bx = lb % nx;
+  lb /= nx;
+  const int by = lb % ny;
+  lb /= ny;
+  const int b = lb / c.n_phase, ph = lb % c.n_phase;
   const int Tin = c.in_len[b], Tout = c.out_len[b];
   const int oo = c.off_out[ph];
   const int r_lo = oo >= 0 ? 0 : (-oo + c.s_out - 1) / c.s_out;
   const int r_hi = Tout - 1 - oo < 0 ? -1 : (Tout - 1 - oo) / c.s_out;
-  const int r0 = r_lo + blockIdx.x * 32;
+  const int r0 = r_lo + bx * 32;
   if (r0 > r_hi) return;  // the whole workgroup leaves together
-  const int co0 = blockIdx.y * (NB * 32);
-  const float* xb = c.x + (size_t)c.in_off[b] * c.ldx;
-  const int cin_pad = (c.Cin + 63) & ~63, nch = cin_pad / 64;
-  // rows co0 .. co0 + NB * 32 - 1 exist: the weights are padded to 64 output channels
-  const bf16_t* wph = wbf + ((size_t)ph * ((c.Cout + 63) & ~63) + co0) * c.taps * cin_pad;
+  const int co0 = by * (NB * 32);
+  const int cin_pad = (c.Cin + 63) & ~63, nch = cin_pad / 64, cpr = cin_pad / 8, rs = cw_stride(c.Cin);
   const int NS = c.taps * nch;
   const int s0 = w * NS / CS_WAVES, s1 = (w + 1) * NS / CS_WAVES;  // this wave's steps (possibly none)
-  const int wr = lane >> 3, wc = lane & 7;    // weight loads: row i * 8 + wr, 16-byte chunk wc
-  const int xr = lane >> 4, xc = lane & 15;   // activation loads: row i * 4 + xr, channels xc * 4 .. + 3
 
-  // step st: tap j = st / nch, input channels cc .. cc + 63 with cc = (st % nch) * 64
-  auto load = [&](int st, float4 (&xv)[8], u32x4 (&wv)[4 * NB]) {
-    const int j = st / nch, cc = (st - j * nch) * 64;
+  // fragments of this wave's steps, in step order: block co0 / 32 + jj, step st, 16-channel slice kk
+  constexpr int DEPTH = 4 / NB;  // steps in flight
+  const size_t blk = (size_t)NS * 4 * 512;
+  const bf16_t* wfr = c.wfr + ((size_t)ph * (((c.Cout + 63) & ~63) / 32) + co0 / 32) * blk + lane * 8;
+  u32x4 wv[DEPTH][NB][4];
+  auto load = [&](int st, u32x4 (&v)[NB][4]) {
 #pragma unroll
-    for (int i = 0; i < 4 * NB; ++i)
-      wv[i] = *(const u32x4*)(wph + ((size_t)(i * 8 + wr) * c.taps + j) * cin_pad + cc + wc * 8);
-    const int ch = cc + xc * 4;
+    for (int jj = 0; jj < NB; ++jj)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = r0 + i * 4 + xr, in_row = r + j * c.d_in + c.off_in[ph];
-      const bool rok = r <= r_hi && in_row >= 0 && in_row < Tin;
-      const float* xp = xb + (size_t)(rok ? in_row : 0) * c.ldx + ch;
-      if (rok && ch + 3 < c.Cin) xv[i] = *(const float4*)xp;
-      else {
-        float t[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] = (rok && ch + u < c.Cin) ? xp[u] : 0.f;
-        xv[i] = make_float4(t[0], t[1], t[2], t[3]);
-      }
-    }
+      for (int kk = 0; kk < 4; ++kk) v[jj][kk] = *(const u32x4*)(wfr + jj * blk + ((size_t)st * 4 + kk) * 512);
   };
-  // activation (zero inputs stay zero: the padding rows and channels of the reference's zero-padded conv), bf16, slab,
-  // fragments, MFMAs
-  auto mma = [&](int st, const float4 (&xv)[8], const u32x4 (&wv)[4 * NB], f32x16 (&acc)[NB]) {
-    const int j = st / nch, cc = (st - j * nch) * 64, ch = cc + xc * 4;
-    float al[4] = {0.f, 0.f, 0.f, 0.f}, iv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (c.pre == PRE_SNAKE) {
-      if (ch + 3 < c.Cin) {
-        const float4 a4 = *(const float4*)(c.alpha + ch), i4 = *(const float4*)(c.inv + ch);
-        al[0] = a4.x; al[1] = a4.y; al[2] = a4.z; al[3] = a4.w;
-        iv[0] = i4.x; iv[1] = i4.y; iv[2] = i4.z; iv[3] = i4.w;
-      } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          al[u] = ch + u < c.Cin ? c.alpha[ch + u] : 0.f;
-          iv[u] = ch + u < c.Cin ? c.inv[ch + u] : 0.f;
+  for (int q = 0; q < DEPTH; ++q)
+    if (s0 + q < s1) load(s0 + q, wv[q]);
+
+  // the slab: input rows in0 .. in0 + nr - 1 of the item (zero outside it: the zero-padded conv's padding), activated
+  const int adil = c.d_in < 0 ? -c.d_in : c.d_in, span = (c.taps - 1) * adil;
+  const int in0 = r0 + c.off_in[ph] - (c.d_in < 0 ? span : 0), nr = 32 + span;
+  {
+    const int rpp = 64 * CS_WAVES / cpr, chunk = tid % cpr, sr = tid / cpr, ch = chunk * 8;
+    float al[8], iv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const bool ok = c.pre == PRE_SNAKE && ch + u < c.Cin;
+      al[u] = ok ? c.alpha[ch + u] : 0.f;
+      iv[u] = ok ? c.inv[ch + u] : 0.f;
+    }
+    const float* xb = c.x + (size_t)c.in_off[b] * c.ldx;
+    constexpr int UN = 2;  // rows in flight per thread
+    for (int base = sr; base < nr; base += UN * rpp) {
+      float v[UN][8];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        const int row = base + u * rpp, in_row = in0 + row;
+        const bool ok = sr < rpp && row < nr && in_row >= 0 && in_row < Tin;
+        const float* xp = xb + (size_t)(ok ? in_row : 0) * c.ldx + ch;
+        if (ok && ch + 7 < c.Cin) {
+          const float4 a = *(const float4*)xp, d = *(const float4*)(xp + 4);
+          v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
+          v[u][4] = d.x; v[u][5] = d.y; v[u][6] = d.z; v[u][7] = d.w;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[u][e] = ok && ch + e < c.Cin ? xp[e] : 0.f;
         }
       }
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        const int row = base + u * rpp, in_row = in0 + row;
+        const bool ok = in_row >= 0 && in_row < Tin;
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = ok && ch + e < c.Cin ? pre_fast(v[u][e], c.pre, c.slope, al[e], iv[e]) : 0.f;
+        if (sr < rpp && row < nr)
+          wlds[row * rs + (chunk ^ ((row >> 1) & 7))] = make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
+      }
     }
-    u32x4* sl = slab[w];
-#pragma unroll
-    for (int i = 0; i < 4 * NB; ++i) {
-      const int r = i * 8 + wr;
-      sl[r * 8 + (wc ^ ((r >> 1) & 7))] = wv[i];
-    }
-    u32x2* sx = (u32x2*)(sl + NB * 256);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int rr = i * 4 + xr, r = r0 + rr, in_row = r + j * c.d_in + c.off_in[ph];
-      const bool rok = r <= r_hi && in_row >= 0 && in_row < Tin;
-      const float v[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
-      float o[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) o[u] = (rok && ch + u < c.Cin) ? pre_fast(v[u], c.pre, c.slope, al[u], iv[u]) : 0.f;
-      u32x2 pk;
-      pk.x = pack2(o[0], o[1]);
-      pk.y = pack2(o[2], o[3]);
-      sx[(rr * 8 + ((xc >> 1) ^ ((rr >> 1) & 7))) * 2 + (xc & 1)] = pk;
-    }
-    u32x4 xf[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) xf[kk] = sl[NB * 256 + cl * 8 + ((h * 4 + kk) ^ ((cl >> 1) & 7))];
-#pragma unroll
-    for (int jj = 0; jj < NB; ++jj) {
-      u32x4 wf[4];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) wf[kk] = sl[(jj * 32 + cl) * 8 + ((h * 4 + kk) ^ ((cl >> 1) & 7))];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        acc[jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wf[kk]), __builtin_bit_cast(bf16x8, xf[kk]), acc[jj], 0, 0, 0);
-    }
-  };
+  }
+  __syncthreads();
 
   f32x16 acc[NB];
 #pragma unroll
   for (int jj = 0; jj < NB; ++jj)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[jj][i] = 0.f;
-  float4 xa[8], xb2[8];
-  u32x4 wa[4 * NB], wb2[4 * NB];
-  // two register sets named at compile time: the loop runs two steps per pass
-  if (s0 < s1) load(s0, xa, wa);
-  for (int st = s0; st < s1; st += 2) {
-    if (st + 1 < s1) load(st + 1, xb2, wb2);
-    mma(st, xa, wa, acc);
-    if (st + 1 < s1) {
-      if (st + 2 < s1) load(st + 2, xa, wa);
-      mma(st + 1, xb2, wb2, acc);
+  int j = s0 / nch, cc = s0 - j * nch;  // tap and chunk of the next step
+  for (int st = s0; st < s1; st += DEPTH) {
+#pragma unroll
+    for (int q = 0; q < DEPTH; ++q) {
+      if (st + q < s1) {
+        const int row = cl + (c.d_in < 0 ? c.taps - 1 - j : j) * adil;
+        const uint4* xr = wlds + row * rs + cc * 8;
+        const int key = (row >> 1) & 7;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const bf16x8 xf = as_bf16x8(xr[(kk * 2 + h) ^ key]);
+#pragma unroll
+          for (int jj = 0; jj < NB; ++jj)
+            acc[jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wv[q][jj][kk]), xf, acc[jj], 0, 0, 0);
+        }
+        if (++cc == nch) cc = 0, ++j;
+        if (st + q + DEPTH < s1) load(st + q + DEPTH, wv[q]);
+      }
     }
   }
-  float4* red = (float4*)slab[w];  // [block jj][quad q][lane]; the wave's own slab (its LDS accesses complete in order)
+  __syncthreads();  // every wave has read the slab
+  float4* red = (float4*)wlds + w * (NB * 256);  // [block jj][quad q][lane]
 #pragma unroll
   for (int jj = 0; jj < NB; ++jj)
 #pragma unroll
@@ -1127,10 +1146,11 @@ __global__ void __launch_bounds__(64 * CS_WAVES) conv_bf16_split_kernel(ConvDesc
   // one float4 (four channels of one row) per thread, summed over the waves in order
   if (tid >= NB * 256) return;
   const int jj = tid >> 8, q = (tid >> 6) & 3, l = tid & 63;
-  float4 sum = ((const float4*)slab[0])[(jj * 4 + q) * 64 + l];
+  const float4* blk0 = (const float4*)wlds + (jj * 4 + q) * 64 + l;
+  float4 sum = blk0[0];
 #pragma unroll
   for (int x = 1; x < CS_WAVES; ++x) {
-    const float4 v = ((const float4*)slab[x])[(jj * 4 + q) * 64 + l];
+    const float4 v = blk0[x * (NB * 256)];
     sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
   }
   // lane l of the MFMA holds output row r0 + l % 32 and channels co0 + jj * 32 + q * 8 + (l / 32) * 4 + 0..3
@@ -1448,6 +1468,25 @@ __global__ void __launch_bounds__(256) snake_kernel(const float4* x, int C4, lon
 }
 
 // rows 1.. of each item's ups output were written one row down; row 0 = input row 1 (ReflectionPad1d((1, 0)))
+// the mean of a stage's three ResBlock outputs, in the running sum's order: ((a + b) + c) / 3
+__global__ void __launch_bounds__(256) mean3_kernel(const float4* a, const float4* b, const float4* c, float4* y, long n4) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const float4 p = a[i], q = b[i], r = c[i];
+  y[i] = make_float4(__fdiv_rn(__fadd_rn(__fadd_rn(p.x, q.x), r.x), 3.f), __fdiv_rn(__fadd_rn(__fadd_rn(p.y, q.y), r.y), 3.f),
+                     __fdiv_rn(__fadd_rn(__fadd_rn(p.z, q.z), r.z), 3.f), __fdiv_rn(__fadd_rn(__fadd_rn(p.w, q.w), r.w), 3.f));
+}
+
+// the last stage's input: row 0 of an item is the reflection of its row 2, then the source branch is added (y != x)
+__global__ void __launch_bounds__(256) reflect_add_kernel(const float4* x, const float4* src, float4* y, int C4, const int* off, const int* len) {
+  const int b = blockIdx.y;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long)len[b] * C4) return;
+  const size_t base = (size_t)off[b] * C4;
+  const float4 v = x[base + i + (i < C4 ? 2 * C4 : 0)], s = src[base + i];
+  y[base + i] = make_float4(__fadd_rn(v.x, s.x), __fadd_rn(v.y, s.y), __fadd_rn(v.z, s.z), __fadd_rn(v.w, s.w));
+}
+
 __global__ void reflect_kernel(float* x, int C, const int* off, int n_items) {
   const int it = blockIdx.y;
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1459,6 +1498,20 @@ __global__ void reflect_kernel(float* x, int C, const int* off, int n_items) {
 inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
 }  // namespace
+
+hipError_t mean3_rows(const float* a, const float* b, const float* c, float* y, long n, hipStream_t st) {
+  if (n % 4) return hipErrorInvalidValue;
+  if (n > 0) hipLaunchKernelGGL(mean3_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, st, (const float4*)a, (const float4*)b, (const float4*)c, (float4*)y, n / 4);
+  return hipGetLastError();
+}
+
+hipError_t reflect_add_rows(const float* x, const float* src, float* y, int C, const int* off, const int* len, int n_items, int max_rows,
+                            hipStream_t st) {
+  if (C % 4) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(reflect_add_kernel, dim3((unsigned)(((long)max_rows * (C / 4) + 255) / 256), n_items), dim3(256), 0, st, (const float4*)x,
+                     (const float4*)src, (float4*)y, C / 4, off, len);
+  return hipGetLastError();
+}
 
 hipError_t snake_rows(const float* x, int C, long rows, const float* alpha, const float* inv, float* y, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
@@ -1523,26 +1576,60 @@ size_t conv_bf16_lds(int BM) {
   return slab > epi ? slab : epi;
 }
 
+bool conv_bf16_window_fits(const ConvDesc& c, int max_rows) {
+  const int span = (c.taps - 1) * (c.d_in < 0 ? -c.d_in : c.d_in);
+  return c.wfr && c.s_in == 1 && c.ldx % 4 == 0 && c.ldy % 4 == 0 && ((size_t)c.x & 15) == 0 && span <= HB_MAXSPAN && c.epi != EPI_SNAKE &&
+         c.n_phase >= 1 && c.n_phase <= 8 && (size_t)(32 + span) * cw_stride(c.Cin) * sizeof(uint4) <= CW_LDS &&
+         (long)cdiv(max_rows, 128) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase < 128;
+}
+
+hipError_t conv_bf16_window(const ConvDesc* c, const int* max_rows, int n, hipStream_t st) {
+  if (n < 1 || n > CONV_BATCH) return hipErrorInvalidValue;
+  long t32 = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!conv_bf16_window_fits(c[i], max_rows[i])) return hipErrorInvalidValue;
+    t32 += (long)cdiv(max_rows[i], 32) * cdiv(c[i].Cout, 32) * c[i].n_items * c[i].n_phase;
+  }
+  // 32 output channels per workgroup where that grid is about one workgroup per CU, else 64: they halve the slabs
+  // filled and activated (58-frame window: 685 us a call; with 32 channels up to 768 workgroups 698, always 825)
+  const int nb = t32 <= 300 ? 1 : 2;
+  ConvBatch cb;
+  cb.n = n;
+  int at = 0;
+  size_t lds = (size_t)CS_WAVES * nb * 256 * sizeof(float4);
+  for (int i = 0; i < CONV_BATCH; ++i) {
+    cb.d[i] = c[i < n ? i : 0];
+    cb.start[i] = at;
+    cb.nx[i] = i < n ? cdiv(max_rows[i], 32) : 1;
+    if (i >= n) continue;
+    at += cb.nx[i] * cdiv(c[i].Cout, 32 * nb) * c[i].n_items * c[i].n_phase;
+    const int adil = c[i].d_in < 0 ? -c[i].d_in : c[i].d_in;
+    lds = std::max(lds, (size_t)(32 + (c[i].taps - 1) * adil) * cw_stride(c[i].Cin) * sizeof(uint4));
+  }
+  cb.start[CONV_BATCH] = at;
+  static const hipError_t attr = [] {  // once per process (thread-safe initialisation)
+    hipError_t e = hipFuncSetAttribute((const void*)conv_bf16_window_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, CW_LDS);
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)conv_bf16_window_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, CW_LDS);
+    return e;
+  }();
+  if (attr != hipSuccess) return attr;
+  if (nb == 1) hipLaunchKernelGGL(conv_bf16_window_kernel<1>, dim3(at), dim3(64 * CS_WAVES), lds, st, cb);
+  else hipLaunchKernelGGL(conv_bf16_window_kernel<2>, dim3(at), dim3(64 * CS_WAVES), lds, st, cb);
+  return hipGetLastError();
+}
+
 hipError_t conv_bf16(const ConvDesc& c, const bf16_t* wbf, int max_rows, hipStream_t st) {
   if (c.n_items <= 0 || max_rows <= 0) return hipSuccess;
   if (c.epi == EPI_SNAKE) return hipErrorInvalidValue;  // fp32 convs only
   if (c.n_phase < 1 || c.n_phase > 8 || c.s_in != 1 || c.ldx % 4 || c.ldy % 4) return hipErrorInvalidValue;
   const int span = (c.taps - 1) * (c.d_in < 0 ? -c.d_in : c.d_in);
   if (span > HB_MAXSPAN) return hipErrorInvalidValue;
-  // 512-row tiles when there are enough of them for the chip, 128 when those fill at least half of it, else 32-row
-  // tiles with the taps split over the waves
+  // 512-row tiles when there are enough of them for the chip, 128 when those fill at least half of it, else the window
+  // kernel's 32-row tiles
   const long tiles512 = (long)cdiv(max_rows, 512) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase;
-  const long tiles128 = (long)cdiv(max_rows, 128) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase;
-  if (tiles128 < 128) {
-    // 32 output channels per workgroup while that grid fits the chip in one round, else 64
-    const long t32 = (long)cdiv(max_rows, 32) * cdiv(c.Cout, 32) * c.n_items * c.n_phase;
-    if (t32 <= 256) {
-      dim3 grid(cdiv(max_rows, 32), cdiv(c.Cout, 32), c.n_items * c.n_phase);
-      hipLaunchKernelGGL(conv_bf16_split_kernel<1>, grid, dim3(64 * CS_WAVES), 0, st, c, wbf);
-    } else {
-      dim3 grid(cdiv(max_rows, 32), cdiv(c.Cout, 64), c.n_items * c.n_phase);
-      hipLaunchKernelGGL(conv_bf16_split_kernel<2>, grid, dim3(64 * CS_WAVES), 0, st, c, wbf);
-    }
+  if (conv_bf16_window_fits(c, max_rows)) {
+    const int mr[1] = {max_rows};
+    return conv_bf16_window(&c, mr, 1, st);
   } else if (!c.wfr) {
     return hipErrorInvalidValue;  // the slab tiles read the fragment-ordered copy
   } else if (tiles512 >= 256) {

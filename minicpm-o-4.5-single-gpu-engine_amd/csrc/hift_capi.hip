@@ -80,9 +80,20 @@ Lens lens_of(const t2w_hift_dims& d, int n, const int* frames) {
 
 struct Bufs {
   float *f0a, *f0b, *f0, *phase, *stft, *X, *XN, *Z, *TMP, *S, *Z2, *post;
+  // window calls: the three ResBlocks' outputs and scratch, the three source branches' outputs and scratch
+  float *wz[3], *wt[3], *ws[3], *wst[3];
 };
 
-size_t carve(const t2w_hift* h, const Lens& L, char* base, Bufs* b) {
+// Calls small enough that the window kernel takes every stage's ResBlock convs (fewer than 128 tiles of 128 rows x 64
+// channels per stage): their ResBlocks run side by side
+bool window_sized(const t2w_hift* h, const Lens& L, int n) {
+  const int cls[3] = {C_S0, C_S1, C_S2};
+  for (int i = 0; i < 3; ++i)
+    if ((long)((L.mx[cls[i]] + 2 + 127) / 128) * ((h->chans[i + 1] + 63) / 64) * n >= 128) return false;
+  return true;
+}
+
+size_t carve(const t2w_hift* h, const Lens& L, int n, char* base, Bufs* b) {
   const t2w_hift_dims& d = h->d;
   size_t big = 0;
   big = std::max(big, (size_t)L.tot[C_T] * d.base);
@@ -104,6 +115,15 @@ size_t carve(const t2w_hift* h, const Lens& L, char* base, Bufs* b) {
   t.S = take(big);
   t.Z2 = take(big);
   t.post = take((size_t)L.tot[C_S2] * (d.n_fft + 2));
+  const int scls[3] = {C_S0, C_S1, C_S2};
+  for (int i = 0; i < 3; ++i) {
+    t.wz[i] = t.wt[i] = t.ws[i] = t.wst[i] = nullptr;
+    if (!window_sized(h, L, n)) continue;
+    t.wz[i] = take(big);
+    t.wt[i] = take(big);
+    t.ws[i] = take((size_t)L.tot[scls[i]] * h->chans[i + 1]);
+    t.wst[i] = take((size_t)L.tot[scls[i]] * h->chans[i + 1]);
+  }
   if (b) *b = t;
   return off * sizeof(float);
 }
@@ -207,6 +227,62 @@ int resblock(const Ctx& x, const t2w_resblock& rb, int k, const float* in, float
   return 0;
 }
 
+// ResBlock `rb` of a window call: its input, class, channels, kernel, output z and scratch tmp (distinct from in)
+struct WindowBlock {
+  const t2w_resblock* rb;
+  const float* in;
+  float *z, *tmp;
+  int C, cls, k;
+};
+
+// The two convs of dilation j of a window call's ResBlock: z = c2(snake(c1(snake(cur)))) + cur, cur the block's input for
+// j = 0 and z (in place: each element is read and written by one thread) after
+void window_convs(const Ctx& x, const WindowBlock& wb, int j, ConvDesc& c1, ConvDesc& c2) {
+  const int dil = x.h->d.res_dilations[j];
+  const float* cur = j == 0 ? wb.in : wb.z;
+  c1 = conv_desc(x, wb.rb->c1[j], cur, wb.C, wb.cls, wb.tmp, wb.C, wb.cls, wb.k, dil, 1, dil * (wb.k - 1) / 2);
+  c1.pre = PRE_SNAKE; c1.alpha = wb.rb->a1[j]; c1.inv = wb.rb->inv1[j];
+  c2 = conv_desc(x, wb.rb->c2[j], wb.tmp, wb.C, wb.cls, wb.z, wb.C, wb.cls, wb.k, 1, 1, (wb.k - 1) / 2);
+  c2.pre = PRE_SNAKE; c2.alpha = wb.rb->a2[j]; c2.inv = wb.rb->inv2[j];
+  c2.res = cur;
+  c2.epi = EPI_RES;
+}
+
+// three independent ResBlocks, each pair of convs of a dilation as one launch for all three
+int window_blocks(const Ctx& x, const WindowBlock (&wb)[3], const char* what) {
+  for (int j = 0; j < 3; ++j) {
+    ConvDesc c1[3], c2[3];
+    int mr[3];
+    for (int i = 0; i < 3; ++i) {
+      window_convs(x, wb[i], j, c1[i], c2[i]);
+      mr[i] = x.L.mx[wb[i].cls] + 2;
+    }
+    H_CHECK(conv_bf16_window(c1, mr, 3, x.st), what);
+    H_CHECK(conv_bf16_window(c2, mr, 3, x.st), what);
+  }
+  return 0;
+}
+
+// whether every ResBlock conv of the call fits the window kernel (bf16 weights, spans, sizes)
+bool window_call(const Ctx& x, const Bufs& B) {
+  if (!x.bf16 || x.fuse == 2 || !B.wz[0]) return false;
+  const t2w_hift_dims& d = x.h->d;
+  const int scls[3] = {C_S0, C_S1, C_S2};
+  for (int i = 0; i < 3; ++i)
+    for (int q = 0; q < 4; ++q) {  // the source ResBlock, then the stage's three
+      const t2w_resblock& rb = q ? x.h->w.res[i * 3 + q - 1] : x.h->w.src_res[i];
+      const WindowBlock wb{&rb, B.XN, B.wz[0], B.wt[0], x.h->chans[i + 1], scls[i], q ? d.res_kernels[q - 1] : d.src_kernels[i]};
+      for (int j = 0; j < 3; ++j) {
+        ConvDesc c1, c2;
+        window_convs(x, wb, j, c1, c2);
+        if (!on_bf16(x, c1) || !on_bf16(x, c2) || wb.C % 4 || !conv_bf16_window_fits(c1, x.L.mx[scls[i]] + 2) ||
+            !conv_bf16_window_fits(c2, x.L.mx[scls[i]] + 2))
+          return false;
+      }
+    }
+  return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -301,7 +377,7 @@ int t2w_hift_plan(const t2w_hift* h, int n, const int* frames, int* plan) {
 
 size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n, const int* frames) {
   if (!h || n <= 0) return 0;
-  return carve(h, lens_of(h->d, n, frames), nullptr, nullptr);
+  return carve(h, lens_of(h->d, n, frames), n, nullptr, nullptr);
 }
 
 int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* plan_dev, const float* mel, const float* noise,
@@ -313,9 +389,9 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
   for (int i = 0; i < n; ++i)
     if (S > class_len(d, C_SMP, frames[i])) return t2w::set_error("source cache longer than a row", hipSuccess);
   if (S > 0 && !cache_source) return t2w::set_error("missing source cache", hipSuccess);
-  if (workspace_bytes < carve(h, x.L, nullptr, nullptr)) return t2w::set_error("hift workspace too small", hipSuccess);
+  if (workspace_bytes < carve(h, x.L, n, nullptr, nullptr)) return t2w::set_error("hift workspace too small", hipSuccess);
   Bufs B;
-  carve(h, x.L, (char*)workspace, &B);
+  carve(h, x.L, n, (char*)workspace, &B);
   const t2w_hift_weights& w = h->w;
   const int harm = d.harmonics + 1, nsrc = d.n_fft + 2;
 
@@ -373,6 +449,25 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
   float* X = B.X;  // stage input (leaky ReLU applied on load)
   float* Sb = B.S;
   const int scls[3] = {C_S0, C_S1, C_S2};
+  // Window calls: a stage's three ResBlocks run side by side (one launch per conv of the three), and so do the three
+  // stages' source branches, which need nothing of the decoder, before it; each value is computed as below.  One
+  // 58-frame window: 62 conv launches -> 29.
+  const bool win = window_call(x, B);
+  auto source_down = [&](int i, float* y) {
+    const int r = i == 0 ? d.up_rates[2] * d.up_rates[1] : (i == 1 ? d.up_rates[2] : 1);
+    ConvDesc c = r == 1 ? conv_desc(x, w.src_down[i], B.stft, STFT_LD, C_S2, y, h->chans[i + 1], scls[i], 1, 1, 1, 0)
+                        : conv_desc(x, w.src_down[i], B.stft, STFT_LD, C_S2, y, h->chans[i + 1], scls[i], 2 * r, 1, r, r / 2);
+    c.w = x.h->src_w32[i];  // padded like the STFT rows
+    return run(x, c, scls[i], "source down");
+  };
+  if (win) {
+    WindowBlock wb[3];
+    for (int i = 0; i < 3; ++i) {
+      if (source_down(i, B.ws[i])) return 1;
+      wb[i] = WindowBlock{&w.src_res[i], B.ws[i], B.ws[i], B.wst[i], h->chans[i + 1], scls[i], d.src_kernels[i]};
+    }
+    if (window_blocks(x, wb, "source resblocks")) return 1;
+  }
   for (int i = 0; i < 3; ++i) {
     const int u = d.up_rates[i], k = d.up_kernels[i], p = (k - u) / 2;
     const int cin = h->chans[i], cout = h->chans[i + 1];
@@ -388,17 +483,30 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
       c.s_in = 1; c.d_in = -1; c.s_out = u; c.n_phase = u;
       for (int ph = 0; ph < u; ++ph) { c.off_in[ph] = 0; c.off_out[ph] = ph - p; }
       c.pre = PRE_LEAKY; c.slope = d.lrelu_slope; c.epi = EPI_STORE; c.n_items = n;
+      if (win && i == 2) c.y = B.TMP;  // reflect_add reads it and writes XN
+      if (win && i < 2) {
+        c.epi = EPI_RES;
+        c.res = B.ws[i];
+      }
       if (run(x, c, i == 2 ? C_S2P : cls, "ups")) return 1;
-      if (i == 2)
+      if (win && i == 2)
+        H_CHECK(timed_launch(T2W_TIMER_HIFT_REFLECT, 12.0 * cout * x.L.tot[cls], x.st,
+                             [&] { return reflect_add_rows(B.TMP, B.ws[2], B.XN, cout, x.off(cls), x.len(cls), n, x.L.mx[cls], x.st); }),
+                "reflection pad and source");
+      else if (i == 2)
         H_CHECK(timed_launch(T2W_TIMER_HIFT_REFLECT, 8.0 * cout * n, x.st, [&] { return reflect_rows(B.XN, cout, x.off(C_S2), n, x.st); }),
                 "reflection pad");
     }
+    if (win) {
+      WindowBlock wb[3];
+      for (int j = 0; j < 3; ++j) wb[j] = WindowBlock{&w.res[i * 3 + j], B.XN, B.wz[j], B.wt[j], cout, cls, d.res_kernels[j]};
+      if (window_blocks(x, wb, "resblocks")) return 1;
+      H_CHECK(mean3_rows(B.wz[0], B.wz[1], B.wz[2], Sb, (long)x.L.tot[cls] * cout, x.st), "resblock mean");
+      std::swap(X, Sb);
+      continue;
+    }
     {  // source branch: downsampling conv of the source STFT, a ResBlock, added into the stage input
-      const int r = i == 0 ? d.up_rates[2] * d.up_rates[1] : (i == 1 ? d.up_rates[2] : 1);
-      ConvDesc c = r == 1 ? conv_desc(x, w.src_down[i], B.stft, STFT_LD, C_S2, B.Z2, cout, cls, 1, 1, 1, 0)
-                          : conv_desc(x, w.src_down[i], B.stft, STFT_LD, C_S2, B.Z2, cout, cls, 2 * r, 1, r, r / 2);
-      c.w = x.h->src_w32[i];  // padded like the STFT rows
-      if (run(x, c, cls, "source down")) return 1;
+      if (source_down(i, B.Z2)) return 1;
       // X (the stage input) is dead once the transposed conv has read it: the ResBlocks' Snake scratch
       if (resblock(x, w.src_res[i], d.src_kernels[i], B.Z2, B.Z2, B.TMP, X, cout, cls, nullptr, 0, B.XN)) return 1;
     }

@@ -32,6 +32,10 @@ hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st);
 // stride-1 / polyphase convs on bf16 MFMA; wbf: bf16 weights [n_phase, Cout padded to 64, taps, Cin padded to 64], and
 // c.wfr the same weights in fragment order (the slab-tile kernels need it)
 hipError_t conv_bf16(const ConvDesc& c, const uint16_t* wbf, int max_rows, hipStream_t st);
+// up to CONV_BATCH independent convs of small grids (each one that fits) in one launch
+constexpr int CONV_BATCH = 3;
+bool conv_bf16_window_fits(const ConvDesc& c, int max_rows);
+hipError_t conv_bf16_window(const ConvDesc* c, const int* max_rows, int n, hipStream_t st);
 // wbf [n_phase, Cout padded to 64, taps, Cin padded to 64] -> out (same size) in MFMA fragment order: for phase ph, output
 // block cb of 32 channels, tap j and input block ib of 16 channels, one 1 KB block whose lane l holds the 8 weights of
 // output channel cb * 32 + l % 32, input channels ib * 16 + (l / 32) * 8 .. + 7 (the A operand of a 32x32x16 MFMA)
@@ -55,6 +59,11 @@ hipError_t stft16(const float* s, const int* smp_off, const int* smp_len, const 
 hipError_t istft16(const float* x, const int* fr_off, const int* fr_len, const int* smp_off, int n_items, int max_smp, const float* win,
                    float limit, float* out, hipStream_t st);
 hipError_t reflect_rows(float* x, int C, const int* off, int n_items, hipStream_t st);
+// y = ((a + b) + c) / 3 over n floats (n % 4 == 0)
+hipError_t mean3_rows(const float* a, const float* b, const float* c, float* y, long n, hipStream_t st);
+// y = x + src over packed rows of C channels, each item's row 0 of x taken from its row 2 (y != x, C % 4 == 0)
+hipError_t reflect_add_rows(const float* x, const float* src, float* y, int C, const int* off, const int* len, int n_items, int max_rows,
+                            hipStream_t st);
 // y = Snake(x) element by element over `rows` packed rows of C channels (C % 4 == 0), y != x
 hipError_t snake_rows(const float* x, int C, long rows, const float* alpha, const float* inv, float* y, hipStream_t st);
 

@@ -165,6 +165,24 @@ def test_resblock_fusion_equals_two_kernels():
             assert torch.equal(outs["auto"], outs["off"]) and e_on < 5e-3
 
 
+@pytest.mark.parametrize("lens,S", [([1], 0), ([58], 3840), ([58, 58], 3840), ([17, 60, 2], 960), ([134], 0), ([137], 0)])
+def test_window_calls_side_by_side(lens, S):
+    """Calls of up to about 135 frames run a stage's three ResBlocks (and the three source branches) side by side on the
+    window kernel, larger ones one after another; against the fused dilations, which never do.  Both round at the same
+    points and differ in the order of fp32 sums, which moves a bf16 rounding now and then (rel-L2 1.5e-3 measured on
+    rows of 1 to 7 frames above; bound 5e-3)."""
+    W = init_hift(HiFTConfig(), seed=6)
+    g = torch.Generator().manual_seed(sum(lens) + S)
+    mel = (torch.randn(sum(lens), 80, generator=g) * 2 - 5).cuda()
+    noise = torch.randn(sum(lens) * 480, 9, generator=g).cuda()
+    cs = (torch.randn(len(lens), S, generator=g) * 0.1).cuda() if S else None
+    outs = [HiFTModel(W, HiFTConfig(), decode_bf16=True, resblock_fusion=f).forward_packed(lens, mel, noise, cs, S)[:2] for f in ("auto", "on")]
+    assert torch.equal(outs[0][1], outs[1][1])
+    e = rel(outs[0][0].cpu(), outs[1][0].cpu())
+    print("window call", lens, S, "rel-L2", e)
+    assert e < 5e-3
+
+
 def test_hift_graphs_equal_eager():
     """Graph replays (one graph per row lengths and source-cache length) equal eager calls bit for bit, replay after
     replay with new inputs, eager work and synchronisations in between; a second key gets its own graph."""
