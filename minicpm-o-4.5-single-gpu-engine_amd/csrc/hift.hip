@@ -1576,18 +1576,18 @@ size_t conv_bf16_lds(int BM) {
   return slab > epi ? slab : epi;
 }
 
-bool conv_bf16_window_fits(const ConvDesc& c, int max_rows) {
+bool conv_bf16_window_fits(const ConvDesc& c, int max_rows, int tiles) {
   const int span = (c.taps - 1) * (c.d_in < 0 ? -c.d_in : c.d_in);
   return c.wfr && c.s_in == 1 && c.ldx % 4 == 0 && c.ldy % 4 == 0 && ((size_t)c.x & 15) == 0 && span <= HB_MAXSPAN && c.epi != EPI_SNAKE &&
          c.n_phase >= 1 && c.n_phase <= 8 && (size_t)(32 + span) * cw_stride(c.Cin) * sizeof(uint4) <= CW_LDS &&
-         (long)cdiv(max_rows, 128) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase < 128;
+         (long)cdiv(max_rows, 128) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase < tiles;
 }
 
 hipError_t conv_bf16_window(const ConvDesc* c, const int* max_rows, int n, hipStream_t st) {
   if (n < 1 || n > CONV_BATCH) return hipErrorInvalidValue;
   long t32 = 0;
   for (int i = 0; i < n; ++i) {
-    if (!conv_bf16_window_fits(c[i], max_rows[i])) return hipErrorInvalidValue;
+    if (!conv_bf16_window_fits(c[i], max_rows[i], CONV_WINDOW_BATCH_TILES)) return hipErrorInvalidValue;
     t32 += (long)cdiv(max_rows[i], 32) * cdiv(c[i].Cout, 32) * c[i].n_items * c[i].n_phase;
   }
   // 32 output channels per workgroup where that grid is about one workgroup per CU, else 64: they halve the slabs
@@ -1624,10 +1624,10 @@ hipError_t conv_bf16(const ConvDesc& c, const bf16_t* wbf, int max_rows, hipStre
   if (c.n_phase < 1 || c.n_phase > 8 || c.s_in != 1 || c.ldx % 4 || c.ldy % 4) return hipErrorInvalidValue;
   const int span = (c.taps - 1) * (c.d_in < 0 ? -c.d_in : c.d_in);
   if (span > HB_MAXSPAN) return hipErrorInvalidValue;
-  // 512-row tiles when there are enough of them for the chip, 128 when those fill at least half of it, else the window
-  // kernel's 32-row tiles
+  // 512-row tiles when there are enough of them for the chip, 128 when those fill it once, else the window kernel's
+  // 32-row tiles
   const long tiles512 = (long)cdiv(max_rows, 512) * cdiv(c.Cout, HB_BN) * c.n_items * c.n_phase;
-  if (conv_bf16_window_fits(c, max_rows)) {
+  if (conv_bf16_window_fits(c, max_rows, CONV_WINDOW_TILES)) {
     const int mr[1] = {max_rows};
     return conv_bf16_window(&c, mr, 1, st);
   } else if (!c.wfr) {

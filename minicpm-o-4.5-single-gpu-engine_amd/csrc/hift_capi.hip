@@ -84,12 +84,11 @@ struct Bufs {
   float *wz[3], *wt[3], *ws[3], *wst[3];
 };
 
-// Calls small enough that the window kernel takes every stage's ResBlock convs (fewer than 128 tiles of 128 rows x 64
-// channels per stage): their ResBlocks run side by side
+// Calls small enough that the window kernel takes every stage's ResBlock convs: their ResBlocks run side by side
 bool window_sized(const t2w_hift* h, const Lens& L, int n) {
   const int cls[3] = {C_S0, C_S1, C_S2};
   for (int i = 0; i < 3; ++i)
-    if ((long)((L.mx[cls[i]] + 2 + 127) / 128) * ((h->chans[i + 1] + 63) / 64) * n >= 128) return false;
+    if ((long)((L.mx[cls[i]] + 2 + 127) / 128) * ((h->chans[i + 1] + 63) / 64) * n >= CONV_WINDOW_BATCH_TILES) return false;
   return true;
 }
 
@@ -275,8 +274,8 @@ bool window_call(const Ctx& x, const Bufs& B) {
       for (int j = 0; j < 3; ++j) {
         ConvDesc c1, c2;
         window_convs(x, wb, j, c1, c2);
-        if (!on_bf16(x, c1) || !on_bf16(x, c2) || wb.C % 4 || !conv_bf16_window_fits(c1, x.L.mx[scls[i]] + 2) ||
-            !conv_bf16_window_fits(c2, x.L.mx[scls[i]] + 2))
+        if (!on_bf16(x, c1) || !on_bf16(x, c2) || wb.C % 4 || !conv_bf16_window_fits(c1, x.L.mx[scls[i]] + 2, CONV_WINDOW_BATCH_TILES) ||
+            !conv_bf16_window_fits(c2, x.L.mx[scls[i]] + 2, CONV_WINDOW_BATCH_TILES))
           return false;
       }
     }

@@ -34,7 +34,12 @@ hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st);
 hipError_t conv_bf16(const ConvDesc& c, const uint16_t* wbf, int max_rows, hipStream_t st);
 // up to CONV_BATCH independent convs of small grids (each one that fits) in one launch
 constexpr int CONV_BATCH = 3;
-bool conv_bf16_window_fits(const ConvDesc& c, int max_rows);
+// A conv is small while 128 x 64 tiles of it number fewer than this: one alone up to about one per CU, three side by
+// side to 300.  Measured (us a call, limits 128 -> these): rows x frames 1x190 1458 -> 1202, 1x300 1945 -> 1667,
+// 2x120 1746 -> 1467, 4x58 1735 -> 1396, 8x58 2549 -> 2040, 16x58 3138 -> 2930; with 300 for one conv alone 2x221 went
+// 2027 -> 2190 (stage 1, 280 tiles)
+constexpr int CONV_WINDOW_TILES = 260, CONV_WINDOW_BATCH_TILES = 300;
+bool conv_bf16_window_fits(const ConvDesc& c, int max_rows, int tiles);
 hipError_t conv_bf16_window(const ConvDesc* c, const int* max_rows, int n, hipStream_t st);
 // wbf [n_phase, Cout padded to 64, taps, Cin padded to 64] -> out (same size) in MFMA fragment order: for phase ph, output
 // block cb of 32 channels, tap j and input block ib of 16 channels, one 1 KB block whose lane l holds the 8 weights of
