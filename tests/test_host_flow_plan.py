@@ -155,3 +155,22 @@ def enc_new(enc, stack):
 
 def lib_calls(enc):
     return _lib.lib().calls
+
+
+def test_ref_pool_counts_duplicates():
+    """A list may name a slot more than once (a trimmed tiled list): every mention counts, a slot goes back to the free
+    stack once, when none is left, and a release too many is refused."""
+    from t2w_amd.flow import RefPool
+
+    p = RefPool(8)
+    ids = p.alloc(3)
+    p.hold([ids[0], ids[0], ids[2]])
+    p.drop(ids)
+    assert p.in_use() == 2 and p.ref.tolist().count(0) == 6
+    p.drop(np.array([ids[0], ids[2]]))
+    assert p.in_use() == 1
+    p.drop([ids[0]])
+    assert p.in_use() == 0 and not p.ref.any()
+    p.drop([])
+    with pytest.raises(RuntimeError):
+        p.drop([ids[1]])
