@@ -184,16 +184,25 @@ __global__ void __launch_bounds__(256) flow_kv_store_kernel(const f16_t* qkv, in
   for (int c = lane * 8; c < 2 * C; c += 512) *(uint4*)(dst + c) = *(const uint4*)(src + c);
 }
 
-// One wave per (32-query tile, head).  MFMA v_mfma_f32_32x32x16_f16 with the scores transposed, S^T = K . Q^T, so a
+// this wave's LDS accesses so far are done (its buffers are its own: no other wave is waited for)
+__device__ __forceinline__ void lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// One wave per (32-query tile, head), or KS of them that take every KS-th key tile each and merge their softmax states
+// through LDS: a wave's serial key tiles (gather by slot, scores, band, softmax) at ~1.5 us each bound the call where the
+// grid leaves CUs idle.  One 28-token window (175 and 350 keys): 15.6 -> 10.9 us per call with eight
+// (the call 459 -> 407 us); four prompts of 75 to 225 tokens 20.7 -> 12.0 (eight) and 19.9 (four, 400-450 keys).  MFMA v_mfma_f32_32x32x16_f16 with the scores transposed, S^T = K . Q^T, so a
 // lane holds 16 keys of its own query (column lane % 32; key rows (r / 4) * 8 + (lane / 32) * 4 + r % 4 of register r)
 // and its partner lane (lane ^ 32) the other 16; O^T += V^T . P^T keeps the output in the same per-query lanes.
 // Positional scores: G^T = Pband . Qv^T over the 64 table rows rb .. rb + 63, rb = L - T + i0 - j0 - 31, the 63
 // relative positions (i - j) + 31 of the tile pair; (key jj, query ii) takes G^T[ii - jj + 31][ii].
-__global__ void __launch_bounds__(64) flow_rel_attn_kernel(RelAttnArgs a) {
+template <int KS>
+__global__ void __launch_bounds__(64 * KS) flow_rel_attn_kernel(RelAttnArgs a) {
   constexpr int GS = 40;                 // row stride of G^T in LDS: conflict-free for the writes and the skewed reads
-  __shared__ float gsh[64 * GS];
-  __shared__ uint4 vsh[32 * 9];          // V tile: 32 key rows of 64 fp16 (8 chunks), row stride 9 chunks
-  const int tile = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+  __shared__ float gall[KS][64 * GS];    // each wave's own
+  __shared__ uint4 vall[KS][32 * 9];     // V tile: 32 key rows of 64 fp16 (8 chunks), row stride 9 chunks
+  const int tile = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float* gsh = gall[wave];
+  uint4* vsh = vall[wave];
   const int s = a.tiles[2 * tile], i0 = a.tiles[2 * tile + 1];
   const int T = a.row_len[s], L = a.kv_len[s], start = a.row_start[s];
   const int* kv = a.kv_idx + a.kv_off[s];
@@ -224,7 +233,7 @@ __global__ void __launch_bounds__(64) flow_rel_attn_kernel(RelAttnArgs a) {
   const float sl2 = a.scale * 1.4426950408889634f;
   const int zero_row = a.rmax - 1, last_row = 2 * a.rmax - 2;
 
-  for (int j0 = 0; j0 < L; j0 += 32) {
+  for (int j0 = 32 * wave; j0 < L; j0 += 32 * KS) {
     // keys (A operand rows): key j0 + col
     half8 kf[4];
     {
@@ -269,7 +278,7 @@ __global__ void __launch_bounds__(64) flow_rel_attn_kernel(RelAttnArgs a) {
       gsh[pr * GS + col] = g0[r];
       gsh[(pr + 32) * GS + col] = g1[r];
     }
-    __syncthreads();
+    lds_fence();
     float sv[16];
     float mx = NEG;
 #pragma unroll
@@ -309,7 +318,33 @@ __global__ void __launch_bounds__(64) flow_rel_attn_kernel(RelAttnArgs a) {
       o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb, o0, 0, 0, 0);
       o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vb, pb, o1, 0, 0, 0);
     }
-    __syncthreads();  // LDS reads done before the next tile's writes
+    lds_fence();  // LDS reads done before the next tile's writes
+  }
+  if constexpr (KS > 1) {
+    // waves 1.. leave (output, max, sum) per lane in their score buffers, wave 0 folds them in in wave order, each
+    // rescaled by 2^(m_w - m*); a wave without tiles brings m = NEG, l = 0 and so a factor 0
+    static_assert(34 * 64 <= 64 * GS, "merge state fits the score buffer");
+    if (wave > 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) { gsh[r * 64 + lane] = o0[r]; gsh[(16 + r) * 64 + lane] = o1[r]; }
+      gsh[32 * 64 + lane] = m;
+      gsh[33 * 64 + lane] = l;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 1; w < KS; ++w) {
+      const float* y = gall[w];
+      const float mg = y[32 * 64 + lane], lg = y[33 * 64 + lane];
+      const float mn = fmaxf(m, mg), fa = __builtin_amdgcn_exp2f(m - mn), fb = __builtin_amdgcn_exp2f(mg - mn);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        o0[r] = o0[r] * fa + y[r * 64 + lane] * fb;
+        o1[r] = o1[r] * fa + y[(16 + r) * 64 + lane] * fb;
+      }
+      l = l * fa + lg * fb;
+      m = mn;
+    }
   }
   if (qi < T) {
     const float inv = 1.0f / l;
@@ -389,7 +424,10 @@ hipError_t flow_kv_store(const f16_t* qkv, int ldq, f16_t* pool, const int* slot
 hipError_t flow_rel_attention(const RelAttnArgs& a, hipStream_t st) {
   if (a.n_tiles <= 0) return hipSuccess;
   if (a.heads <= 0 || a.ldq % 8 || a.rmax < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(flow_rel_attn_kernel, dim3(a.n_tiles, a.heads), dim3(64), 0, st, a);
+  const int wgs = a.n_tiles * a.heads;  // eight waves' buffers fill a CU, four leave room for two workgroups
+  if (wgs < 256) hipLaunchKernelGGL(flow_rel_attn_kernel<8>, dim3(a.n_tiles, a.heads), dim3(512), 0, st, a);
+  else if (wgs < 1024) hipLaunchKernelGGL(flow_rel_attn_kernel<4>, dim3(a.n_tiles, a.heads), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL(flow_rel_attn_kernel<1>, dim3(a.n_tiles, a.heads), dim3(64), 0, st, a);
   return hipGetLastError();
 }
 

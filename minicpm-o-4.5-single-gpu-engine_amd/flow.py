@@ -264,16 +264,18 @@ class FlowEncoder:
             g = {"offs": offs, "arena": torch.zeros(size, dtype=torch.int32, device=self.device),
                  "ws": torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=self.device),
                  "mu": torch.empty(n2, self.cfg.mel, dtype=torch.float32, device=self.device), "graph": None}
-        # the tables and the first key list in one upload, the second list in another: the lists' unused capacity (rmax
-        # keys per row each, never read past a row's length) is not sent
-        offs, kv2 = g["offs"], parts["kv2_idx"]
-        host = np.zeros(offs["kv1_idx"] + parts["kv1_idx"].size, dtype=np.int32)
+        # the key lists go up at their length, from one staging block: their unused capacity (rmax keys per row each, never
+        # read past a row's length) is not sent
+        offs, n_kv2 = g["offs"], parts["kv2_idx"].size
+        end1 = offs["kv1_idx"] + parts["kv1_idx"].size
+        host = np.zeros(end1 + n_kv2, dtype=np.int32)
         for k, v in parts.items():
-            if k != "kv2_idx":
-                v = np.asarray(v)
-                host[offs[k]:offs[k] + v.size] = v
-        _Upload.into(g["arena"], host)
-        _Upload.into(g["arena"][offs["kv2_idx"]:], kv2.astype(np.int32))
+            v, o = np.asarray(v), end1 if k == "kv2_idx" else offs[k]
+            host[o:o + v.size] = v
+        src = torch.from_numpy(host)
+        src = src.pin_memory() if g["arena"].is_cuda else src
+        g["arena"][:end1].copy_(src[:end1], non_blocking=True)
+        g["arena"][offs["kv2_idx"]:offs["kv2_idx"] + n_kv2].copy_(src[end1:], non_blocking=True)
         if g["graph"] is None:
             if self._cap is None:
                 self._cap = torch.cuda.Stream()

@@ -147,3 +147,19 @@ def test_window_graphs_equal_eager(dev):
             if x is not None:
                 e.release(x)
     assert all(e.in_use() == (0, 0, 0) for e in encs)
+
+
+@pytest.mark.parametrize("n", [2, 6, 20])
+def test_key_groups_match_oracle(flow, n):
+    """Prompts of 97 and 17 tokens in one call of n: attention grids of 40 workgroups (eight waves share a query tile's
+    keys), up to 240 and 480 in the two stacks (eight, then four) and 800 to 1,600 (four, then one), rows with fewer key
+    tiles than waves among them."""
+    W, d, enc = flow
+    g = torch.Generator().manual_seed(8)
+    two = [torch.randint(0, d.vocab, (t,), generator=g).tolist() for t in (97, 17)]
+    states, mu, rows, frames = enc.setup([two[i % 2] for i in range(n)])
+    refs = [of.setup(W, d, p)[0] for p in two]
+    for i in (0, 1, n - 2, n - 1):
+        assert rel(mu[rows[i]:rows[i] + frames[i]].t().cpu(), refs[i % 2]) < TOL
+    for st in states:
+        enc.release(st)
