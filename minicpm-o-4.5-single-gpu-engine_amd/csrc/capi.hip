@@ -198,7 +198,7 @@ Defer defer_plan(const t2w_dit_dims& d, int N, int K, const Work& w, bool taps) 
   if (!w.part) return Defer{1, -1};
   const int most = (int)std::min<size_t>(4, w.part_bytes / ((size_t)N * H * 4));
   if (N > GEMM_SMALL_MAX_M) {
-    const RingPlan rp = ring_plan(N, H, K, std::max(most, 1), false);
+    const RingPlan rp = ring_plan(N, H, K, std::max(most, 1), false, false);
     return Defer{rp.cfg < 0 ? 1 : rp.splits, rp.cfg};
   }
   // the conv GEMMs (taps) run on 64-row tiles above 32 tokens (gemm_small_part64), proj and fc2 on 32-row tiles
@@ -292,7 +292,7 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     const bool small_qkv = gemm_small_fits(gq, EPI_QKV);
     GemmArgs gr = gq;
     gr.qk.rfreq = nullptr;
-    const RingPlan rp_qkv = f8 ? RingPlan{-1, 1} : ring_plan(N, 3 * H, H, 1, true);
+    const RingPlan rp_qkv = ring_plan(N, 3 * H, H, 1, true, f8);
     if (!small_qkv && rp_qkv.cfg >= 0 && gemm_ring_fits(gr, EPI_QKV)) {
       T2W_CHECK(gemm_ring(gr, EPI_QKV, rp_qkv.cfg, st), "qkv");
       if (m->g.rope_freq) T2W_CHECK(rope_qk(w.q, kp, a->new_slot, a->tok_abs, m->g.rope_freq, N, H, st), "rope");

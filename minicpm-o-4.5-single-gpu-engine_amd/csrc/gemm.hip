@@ -229,7 +229,7 @@ hipError_t gemm_bf16(const GemmArgs& g, int epi, hipStream_t st, int cfg) {
     return hipErrorInvalidValue;
   if (cfg < 0 && gemm_small_fits(g, epi)) return gemm_small(g, epi, st);
   if (cfg < 0 && epi != EPI_PART && gemm_ring_fits(g, epi)) {
-    const RingPlan rp = ring_plan(g.M, g.N, g.K, 1, epi == EPI_QKV);
+    const RingPlan rp = ring_plan(g.M, g.N, g.K, 1, epi == EPI_QKV, g.w_scale != nullptr);
     if (rp.cfg >= 0) return gemm_ring(g, epi, rp.cfg, st);
   }
   // the tile epilogues store bf16 rows 16 bytes per lane

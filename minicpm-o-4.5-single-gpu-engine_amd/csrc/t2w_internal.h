@@ -84,13 +84,13 @@ hipError_t gemm_small(const GemmArgs& g, int epi, hipStream_t st);
 // whether an EPI_PART call runs on 64-row tiles (taps mode, more than 32 rows, at most 16 64-K steps per split)
 bool gemm_small_part64(const GemmArgs& g);
 
-// Ring-buffered GEMM on 64x64, 128x64 or 128x128 tiles (bf16; gemm_ring.hip).  ring_plan: the cheapest tile shape for a
+// Ring-buffered GEMM on 64x64 to 256x128 tiles (gemm_ring.hip).  ring_plan: the cheapest tile shape for a
 // call of M rows whose sums may be split up to max_splits ways (EPI_PART; 1 for the other epilogues), cfg < 0 when its
 // grids hold more workgroups than it is meant for.  qkv: EPI_QKV (its tile shapes differ).
 struct RingPlan {
   int cfg, splits;
 };
-RingPlan ring_plan(int M, int N, int K, int max_splits, bool qkv);
+RingPlan ring_plan(int M, int N, int K, int max_splits, bool qkv, bool fp8);
 bool gemm_ring_fits(const GemmArgs& g, int epi);
 hipError_t gemm_ring(const GemmArgs& g, int epi, int cfg, hipStream_t st);
 

@@ -174,10 +174,11 @@ def test_gemm_splitk(dev, M, N, K, epi):
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 64, 64), (129, 3072, 128), (191, 72, 192), (193, 1024, 256), (321, 1024, 1024), (449, 1000, 320),
-                                   (1025, 2048, 64), (1300, 1024, 2048), (2049, 1024, 448), (4096, 1024, 128)])
+                                   (1025, 2048, 64), (1300, 1024, 2048), (2049, 1024, 448), (4096, 1024, 128),
+                                   (4200, 1000, 256), (6145, 1024, 192)])
 @pytest.mark.parametrize("epi", [0, 1, 2, 3, 7])
 def test_gemm_ring(dev, M, N, K, epi):
-    """The ring-buffered tiles (64x64, 128x64, 128x128 by shape) at the edges of tiles, of the ring (K of one to eight
+    """The ring-buffered tiles (64x64 to 256x128 by shape) at the edges of tiles, of the ring (K of one to eight
     stages) and of the output columns; dense and, where the epilogue has it, taps (rows of K / 64 64-value frames),
     which read the same values and so give the same bits.  Bounds: one bf16 rounding is at most 2^-9 of a value, one
     fp16 rounding 2^-12, fp32 sums of up to 2048 products stay within 1e-5."""
@@ -505,6 +506,36 @@ def test_gemm_fp8_large_tiles(dev, N, epi):
     if N == 3072:  # the rows of the last partial round (the 256 x 128 tail) on their own
         tail = slice(M - 1536, M)
         assert rel(out[tail].float(), ref[tail]) < 6e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (70, 256, 128), (129, 1024, 384), (1000, 1000, 1152), (2000, 1024, 512), (4200, 1024, 640),
+                                   (6145, 1024, 384)])
+@pytest.mark.parametrize("epi", [0, 2])
+@pytest.mark.parametrize("taps", [False, True])
+def test_gemm_ring_fp8(dev, M, N, K, epi, taps):
+    """The ring-buffered tiles on fp8 at the edges of tiles, of the ring (K of one to nine stages) and of the columns,
+    dense and taps (rows of K / 128 128-value frames), against fp32 matmul of the dequantized operands (bounds as
+    test_gemm_fp8)."""
+    L = _lib.lib()
+    g = torch.Generator().manual_seed(M + N + K + epi)
+    frames = torch.randn(M + K // 128 - 1, 128, generator=g).bfloat16()
+    A = frames if taps else torch.cat([frames[j:j + M] for j in range(K // 128)], 1).contiguous()
+    qa, sa = of.quantize_mx(A)
+    Ad = of.dequantize_mx(qa, sa).to(dev)
+    Ad = torch.cat([Ad[j:j + M] for j in range(K // 128)], 1) if taps else Ad
+    qw, sw = of.quantize_weight(torch.randn(N, K, generator=g) / K ** 0.5)
+    Wd = of.dequantize_weight(qw, sw).to(dev)
+    qa, sa, qw, sw = qa.to(dev), sa.to(dev), qw.to(dev), sw.to(dev)
+    bias, gate = torch.randn(N, generator=g).to(dev), torch.randn(N, generator=g).to(dev)
+    h0 = torch.randn(M, N, generator=g).half().to(dev)
+    out = h0.clone() if epi == 2 else torch.full((M, N), 7.0, device=dev).bfloat16()
+    src = torch.arange(M, dtype=torch.int32, device=dev) if taps else None
+    ld = 128 if taps else K
+    _lib.check(L.t2w_gemm_fp8(qa.data_ptr(), ld, _lib.ptr(src), sa.data_ptr(), ld // 32, qw.data_ptr(), sw.data_ptr(), bias.data_ptr(),
+                              gate.data_ptr() if epi == 2 else None, out.data_ptr(), N, M, N, K, epi, _lib.stream_handle()), "gemm_fp8")
+    torch.cuda.synchronize()
+    ref = Ad @ Wd.t() + bias
+    assert rel(out.float(), h0.float() + gate * ref if epi == 2 else ref) < (1e-3 if epi == 2 else 6e-3)
 
 
 def test_gemm_fp8_taps(dev):
