@@ -186,10 +186,9 @@ GemmArgs gemm8(const uint8_t* A, int lda, const int* a_src, const uint8_t* as, c
 }
 
 // K splits of a deferred GEMM, [N, H] from K, whose result a row kernel finishes (splits < 2: not deferred): at most 4
-// (the row kernels' limit), and the sums must fit the partial area.  Up to 128 rows it runs on the small-row kernel
-// (ring_cfg < 0), with enough workgroups to occupy the 256 CUs: its weights come from HBM, and a workgroup that issues
-// all its loads at once waits less for them than one that keeps three ring stages in flight (in a one-window solve
-// conv 7.1 us against 7.7, proj and fc2 5.6 against 5.8).  Beyond, on the ring tiles.
+// (the row kernels' limit), and the sums must fit the partial area.  proj and fc2 of up to 128 rows run on the small-row
+// kernel's 32-row tiles (ring_cfg < 0), with enough workgroups to occupy the 256 CUs; everything else on the ring tiles
+// (a one-window solve of 13.25 ms: conv1 and conv2 on the ring 13.15, proj and fc2 too 13.39).
 struct Defer {
   int splits, ring_cfg;
 };
@@ -197,20 +196,14 @@ Defer defer_plan(const t2w_dit_dims& d, int N, int K, const Work& w, bool taps) 
   const int H = d.hidden;
   if (!w.part) return Defer{1, -1};
   const int most = (int)std::min<size_t>(4, w.part_bytes / ((size_t)N * H * 4));
-  if (N > GEMM_SMALL_MAX_M) {
+  if (N > GEMM_SMALL_MAX_M || taps) {
     const RingPlan rp = ring_plan(N, H, K, std::max(most, 1), false, false);
     return Defer{rp.cfg < 0 ? 1 : rp.splits, rp.cfg};
   }
-  // the conv GEMMs (taps) run on 64-row tiles above 32 tokens (gemm_small_part64), proj and fc2 on 32-row tiles
-  // (measured faster for them: K = 1024 / 2048 leaves 64-row tiles too few steps per workgroup)
-  const int rows = taps && N > 32 ? 64 : 32;
-  const int tiles = ((N + rows - 1) / rows) * ((H + 31) / 32);
+  const int tiles = ((N + 31) / 32) * ((H + 31) / 32);
   const int S = std::min(most, 256 / tiles);
-  static const int taps_marker = 0;  // gemm_small_fits checks only the presence of a frame id list
   GemmArgs g{};
-  g.M = N; g.N = H; g.ldc = H; g.splits = S; g.tapC = H; g.K = K; g.ldb = K;
-  g.lda = taps ? H : K;
-  g.a_src = taps ? &taps_marker : nullptr;
+  g.M = N; g.N = H; g.ldc = H; g.splits = S; g.K = K; g.ldb = K; g.lda = K;
   return Defer{S >= 2 && gemm_small_fits(g, EPI_PART) ? S : 1, -1};
 }
 

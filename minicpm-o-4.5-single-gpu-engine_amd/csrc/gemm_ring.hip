@@ -1,5 +1,5 @@
-// bf16 MFMA GEMM for calls whose 256-row tile grids would leave most CUs idle: streaming windows (the deferred GEMMs from
-// one window's ~100 rows on), prompt setups, several streams at once, up to a few thousand rows.
+// bf16 and fp8 MFMA GEMM for calls whose 256-row tile grids would leave most CUs idle: the K-split convs of a streaming
+// window, several windows at once, prompt setups, batches of up to about 8,000 rows.
 //
 // Small tiles (64x64, 128x64, 128x128) put a workgroup on every CU; what bounds them is the latency of a K stage, so the
 // stages run through a ring of NS LDS buffers filled by global_load_lds, NS - 1 of them in flight, with one

@@ -385,13 +385,11 @@ struct Tile {
   // loads of stage kt into (la, lb) and, in fp8 mode, its activation scale dwords into sd
   __device__ __forceinline__ void issue(uint4* la, uint4* lb, uint32_t (&sd)[NSC], int kt) const {
     const int k0 = kt * BKE;
-    size_t aoff = (size_t)k0 * ES;
+    const size_t aoff = (size_t)k0 * ES;  // taps: a row's frames follow each other, so K runs on across them
     int srow = 0, sblk = k0 / 32;
-    if (TAPS) {
-      const int tap = k0 / g.tapC;  // a stage never straddles two taps (tapC % BKE == 0)
-      aoff = ((size_t)tap * g.lda + (k0 - tap * g.tapC)) * ES;
-      srow = tap;
-      sblk = (k0 - tap * g.tapC) / 32;
+    if (TAPS && FP8) {  // the scale rows may be further apart
+      srow = k0 / g.tapC;  // a stage never straddles two taps (tapC % BKE == 0)
+      sblk = (k0 - srow * g.tapC) / 32;
     }
     const uint8_t* A = (const uint8_t*)g.A;
     const uint8_t* B = (const uint8_t*)g.B;

@@ -14,7 +14,7 @@ typedef uint16_t f16_t;  // storage type of the fp16 residual stream
 // EPI_GELU_MX8: GELU, then MX fp8 codes to C (bytes, ldc) and block scales to c_scale (N % 32 == 0)
 // EPI_QKV: the attention projection (N = 3 H): q and k rounded to bf16, per-head LayerNorm + affine, q to its token
 // row of q_out, k and v to the token's key slot of the pools (fields qk.*); tile path only
-// EPI_PART (small-row GEMM only): K split over `splits` workgroups per tile, split z writes its fp32 sum without bias
+// EPI_PART (small-row and ring GEMMs): K split over `splits` workgroups per tile, split z writes its fp32 sum without bias
 // to C + z * c_split (rows ldc apart); a row kernel that takes the sums as a Pend finishes the GEMM's epilogue
 // Epilogues.  EPI_RESID_F16: the gated residual C(fp16) = fp16(C + gate * (acc + bias)), the residual stream kept in the
 // reference's fp16 with fp32 arithmetic; EPI_F16: fp16 out.
@@ -33,7 +33,7 @@ struct QkvOut {
 };
 
 struct GemmArgs {
-  const bf16_t* A;     // dense: A[m * lda + k]; taps: A[(a_src[m] + k / tapC) * lda + k % tapC]
+  const bf16_t* A;     // dense: A[m * lda + k]; taps: A[a_src[m] * lda + k], frames of tapC = lda values
   int lda;
   const int* a_src;    // taps mode when non-null
   int tapC;
@@ -81,9 +81,6 @@ bool gemm_splits(const GemmArgs& g);  // whether gemm_bf16 (cfg < 0) takes the s
 constexpr int GEMM_SMALL_MAX_M = 128;
 bool gemm_small_fits(const GemmArgs& g, int epi);
 hipError_t gemm_small(const GemmArgs& g, int epi, hipStream_t st);
-// whether an EPI_PART call runs on 64-row tiles (taps mode, more than 32 rows, at most 16 64-K steps per split)
-bool gemm_small_part64(const GemmArgs& g);
-
 // Ring-buffered GEMM on 64x64 to 256x128 tiles (gemm_ring.hip).  ring_plan: the cheapest tile shape for a
 // call of M rows whose sums may be split up to max_splits ways (EPI_PART; 1 for the other epilogues), cfg < 0 when its
 // grids hold more workgroups than it is meant for.  qkv: EPI_QKV (its tile shapes differ).
