@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(256) conv_f32_kernel(ConvDesc c) {
 }
 
 // The same fp32 convolution with its operands copied straight into LDS (global_load_lds_dwordx4, no register staging
-// and no LDS stores), for Cin a multiple of 32 and 16-byte rows.  A stage is one tap and 32 input channels: 128
+// and no LDS stores), for Cin a multiple of 32 and 16-byte rows.  A stage is one tap and 32 input channels: BM
 // activation rows and 32 WN weight rows of 128 bytes, 16-byte chunks XOR-swizzled by (row / 2) % 8; the lanes of an
 // instruction name the logical chunk that lands in their physical slot.  Rows outside the item (zero padding) and
 // output channels past Cout fetch a 16-byte zero block instead.  A fragment read of 16 bytes gives a lane four K
@@ -388,19 +388,25 @@ __global__ void __launch_bounds__(256) conv_f32_kernel(ConvDesc c) {
 // fragment after the read (zero rows stay zero); Snake convs take conv_f32_kernel (evaluated once per element and stage
 // there, not once per element, tap and wave).  Two LDS stages, separate objects, the K loop unrolled by two: the loads
 // of stage s + 1 are issued before the MFMAs of stage s.
+//
+// Bound by the fp32 matrix rate (157 TFLOP/s).  64 x 64 tiles, four workgroups to a CU, where 128 x 64 ones came two to
+// a CU: with grids of one to three rounds the last round and each workgroup's fill and epilogue left 40% of the rate
+// unused.  Strict fp32, six rows of 50 to 400 frames 15.1 -> 11.7 ms, twelve of 200 to 400 29.8 -> 25.6, two of 100 to
+// 200 5.7 -> 4.1; reference split, sixteen of 50 to 400 6.69 -> 6.43; the same bits.  (Outputs of at most 32 channels
+// keep 128 rows: a wave then owns 32 of them.)
 __device__ __align__(16) float conv_zero16[4];  // never written: the load source of padding rows
 
 __device__ __forceinline__ int fswz(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-template <int WN, int PRE>
-__global__ void __launch_bounds__(256, 2) conv_f32_dma_kernel(ConvDesc c) {
-  constexpr int BN = 32 * WN, WM = 4 / WN, WTM = F_BM / WM, TM = WTM / 32;
-  constexpr int RA = F_BM / 8, NB = RA + BN / 8, PW = NB / 4;  // 8-row load blocks: activations, all, per wave
+template <int BM, int WN, int PRE>
+__global__ void __launch_bounds__(256, BM == 64 ? 4 : 2) conv_f32_dma_kernel(ConvDesc c) {
+  constexpr int BN = 32 * WN, WM = 4 / WN, WTM = BM / WM, TM = WTM / 32;
+  constexpr int RA = BM / 8, NB = RA + BN / 8, PW = NB / 4;  // 8-row load blocks: activations, all, per wave
   static_assert(NB % 4 == 0, "load blocks per wave");
   static_assert(PRE == PRE_NONE || PRE == PRE_LEAKY, "Snake convs take the register-staged kernel (or Snake out of the conv)");
-  __shared__ uint4 sA0[F_BM * 8], sA1[F_BM * 8], sB0[BN * 8], sB1[BN * 8];
+  __shared__ uint4 sA0[BM * 8], sA1[BM * 8], sB0[BN * 8], sB1[BN * 8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int b = blockIdx.z / c.n_phase, ph = blockIdx.z % c.n_phase;
@@ -408,7 +414,7 @@ __global__ void __launch_bounds__(256, 2) conv_f32_dma_kernel(ConvDesc c) {
   const int oo = c.off_out[ph];
   const int r_lo = oo >= 0 ? 0 : (-oo + c.s_out - 1) / c.s_out;
   const int r_hi = Tout - 1 - oo < 0 ? -1 : (Tout - 1 - oo) / c.s_out;
-  const int r0 = r_lo + blockIdx.x * F_BM;
+  const int r0 = r_lo + blockIdx.x * BM;
   if (r0 > r_hi) return;
   const int co0 = blockIdx.y * BN;
   const int Cin = c.Cin, Cout = c.Cout, taps = c.taps, ldx = c.ldx, d_in = c.d_in;
@@ -431,8 +437,8 @@ __global__ void __launch_bounds__(256, 2) conv_f32_dma_kernel(ConvDesc c) {
       rbase[p] = co0 + trow;
     }
   }
-  auto issue = [&](uint4* dA, uint4* dB, int s) __attribute__((always_inline)) {
-    const int j = s / nck, ci = (s - j * nck) * 32;
+  int j = 0, ci = 0;  // tap and first input channel of the next stage to copy
+  auto issue = [&](uint4* dA, uint4* dB) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < PW; ++p) {
       const int blk = wave + 4 * p;
@@ -448,6 +454,8 @@ __global__ void __launch_bounds__(256, 2) conv_f32_dma_kernel(ConvDesc c) {
       }
       __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)dst, 16, 0, 0);
     }
+    ci += 32;
+    if (ci == Cin) ci = 0, ++j;
   };
   f32x16 acc[TM];
 #pragma unroll
@@ -477,16 +485,16 @@ __global__ void __launch_bounds__(256, 2) conv_f32_dma_kernel(ConvDesc c) {
         for (int i = 0; i < TM; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[m], a[i][m], acc[i], 0, 0, 0);
     }
   };
-  issue(sA0, sB0, 0);
+  issue(sA0, sB0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   for (int s = 0; s < S; s += 2) {
-    if (s + 1 < S) issue(sA1, sB1, s + 1);
+    if (s + 1 < S) issue(sA1, sB1);
     compute(sA0, sB0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (s + 1 < S) {
-      if (s + 2 < S) issue(sA0, sB0, s + 2);
+      if (s + 2 < S) issue(sA0, sB0);
       compute(sA1, sB1);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -1545,15 +1553,15 @@ hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st) {
   // the DMA-staged kernel: 32-channel K stages and 16-byte rows (activations and weights)
   if (c.Cin % 32 == 0 && c.ldx % 4 == 0 && ((size_t)c.x & 15) == 0 && ((size_t)c.w & 15) == 0 &&
       (c.pre == PRE_NONE || c.pre == PRE_LEAKY)) {
-    const int wn = c.Cout <= 32 ? 1 : 2;
-    dim3 grid(cdiv(max_rows, F_BM), cdiv(c.Cout, 32 * wn), c.n_items * c.n_phase);
-#define T2W_FD(W, P) hipLaunchKernelGGL((conv_f32_dma_kernel<W, P>), grid, dim3(256), 0, st, c)
+    const int wn = c.Cout <= 32 ? 1 : 2, bm = wn == 1 ? F_BM : 64;
+    dim3 grid(cdiv(max_rows, bm), cdiv(c.Cout, 32 * wn), c.n_items * c.n_phase);
+#define T2W_FD(M, W, P) hipLaunchKernelGGL((conv_f32_dma_kernel<M, W, P>), grid, dim3(256), 0, st, c)
     if (wn == 1) {
-      if (c.pre == PRE_NONE) T2W_FD(1, PRE_NONE);
-      else T2W_FD(1, PRE_LEAKY);
+      if (c.pre == PRE_NONE) T2W_FD(F_BM, 1, PRE_NONE);
+      else T2W_FD(F_BM, 1, PRE_LEAKY);
     } else {
-      if (c.pre == PRE_NONE) T2W_FD(2, PRE_NONE);
-      else T2W_FD(2, PRE_LEAKY);
+      if (c.pre == PRE_NONE) T2W_FD(64, 2, PRE_NONE);
+      else T2W_FD(64, 2, PRE_LEAKY);
     }
 #undef T2W_FD
     return hipGetLastError();
