@@ -255,7 +255,8 @@ int t2w_flow_speaker(const t2w_flow* m, const float* spk, float* out, int R, voi
  * stream, fp16 as the reference's activations, fp32 arithmetic), 3: fp32 out, 7: fp16 out.
  * a_src non-null: conv taps mode, A row m = frames a_src[m] .. a_src[m] + K / lda - 1 of A (rows lda wide).
  * Calls of at most 128 rows (K <= 3072, ldc % 4 == 0) run as one kernel that splits K over the waves of a workgroup;
- * larger ones on the tile GEMM (16-bit outputs: ldc % 8 == 0 and C 16-byte aligned there). */
+ * larger ones on the ring tiles (64x64 to 256x128) where those are the faster ones for the shape, else on the tile GEMM
+ * (16-bit outputs: ldc % 8 == 0 and C 16-byte aligned on both). */
 int t2w_gemm_bf16(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate,
                   void* C, int ldc, int M, int N, int K, int epi, void* stream);
 /* t2w_gemm_bf16 with an explicit tile configuration (-1: chosen by shape; 0: 128x128 of 4 waves, 1: 256x256 of
@@ -263,8 +264,9 @@ int t2w_gemm_bf16(const void* A, int lda, const int* a_src, const void* W, const
  * K % 64 == 0, lda % 8 == 0 (taps mode: lda % 64 == 0). */
 int t2w_gemm_bf16_tile(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate,
                        void* C, int ldc, int M, int N, int K, int epi, int tile, void* stream);
-/* t2w_gemm_bf16 with a workspace for split-K partials (256-byte aligned; up to splits x M x N fp32): a call whose tile
- * grid would leave most CUs idle (few rows) splits K over ~512 waves and reduces the partials in a fixed order. */
+/* t2w_gemm_bf16 with a workspace for split-K partials (256-byte aligned; up to splits x M x N fp32): a call that
+ * neither the small-row kernel nor the ring tiles take (16-bit output rows that are not 16-byte aligned) and whose tile
+ * grid would leave most CUs idle splits K over ~512 waves and reduces the partials in a fixed order. */
 int t2w_gemm_bf16_ws(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate,
                      void* C, int ldc, int M, int N, int K, int epi, void* workspace, size_t workspace_bytes,
                      void* stream);

@@ -191,6 +191,7 @@ hipError_t launch_epi(const GemmArgs& g, int cfg, hipStream_t st) {
 
 }  // namespace
 
+// the tile for calls that the ring tiles do not take (ring_plan: they cost less up to a few thousand rows)
 int pick_cfg(const GemmArgs& g) {
   // 256x256 tiles once there are enough rows to fill them (bf16 and fp8 alike).  qkv (N = 3072) took 256x128 while its
   // epilogue wrote 4 columns per lane (105 us vs 114 at 12800 rows); with 16-byte stores 256x256 is the faster one

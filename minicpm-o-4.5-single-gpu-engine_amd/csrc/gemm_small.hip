@@ -9,7 +9,7 @@
 // (deterministic) and the epilogue (bias, GELU, gated fp32 residual) writes four consecutive columns per lane.
 //
 // A workgroup moves its W and activation rows through one CU, and a CU's load throughput (not HBM) is what bounds
-// these calls: ~100 rows x K = 3072 (conv taps) is 384 KB per workgroup on 128 CUs.  EPI_PART therefore also splits K
+// these calls: ~100 rows x K = 2048 (fc2) is 256 KB per workgroup on 128 CUs.  EPI_PART therefore also splits K
 // over g.splits workgroups per tile (grid z), so that all CUs share the bytes, and leaves the sum of the splits, the
 // bias and the gated residual to the row kernel that reads the result next (Pend).
 //
