@@ -1284,6 +1284,94 @@ __global__ void __launch_bounds__(64 * CS_WAVES) conv_f32_split_kernel(ConvDesc 
   else conv_epilogue_part<true>(c, orow, co0 + cn, ncols - cn, sum);
 }
 
+// conv_f32_split_kernel on 16 output rows x 16 output channels (v_mfma_f32_16x16x4f32; lane group g = lane / 16 supplies
+// channels g * 8 + u of MFMA u on both sides): four times the workgroups, each with half the loads, and a quarter of
+// the MFMAs.  On 32 x 32 tiles a 58-frame window's f0 convs were 32 workgroups, an eighth of the CUs, each bound
+// by its own chain of loads and MFMAs: 20.7 -> 12.3 us per conv, the whole call 683 -> 608 us.
+__global__ void __launch_bounds__(64 * CS_WAVES) conv_f32_split16_kernel(ConvDesc c) {
+  __shared__ float4 red[CS_WAVES][64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, cl = lane & 15;
+  const int b = blockIdx.z / c.n_phase, ph = blockIdx.z % c.n_phase;
+  const int Tin = c.in_len[b], Tout = c.out_len[b];
+  const int oo = c.off_out[ph];
+  const int r_lo = oo >= 0 ? 0 : (-oo + c.s_out - 1) / c.s_out;
+  const int r_hi = Tout - 1 - oo < 0 ? -1 : (Tout - 1 - oo) / c.s_out;
+  const int r0 = r_lo + blockIdx.x * 16;
+  if (r0 > r_hi) return;  // the whole workgroup leaves together
+  const int co0 = blockIdx.y * 16;
+  const float* xb = c.x + (size_t)c.in_off[b] * c.ldx;
+  const int nch = (c.Cin + 31) / 32, NS = c.taps * nch;
+  const int s0 = w * NS / CS_WAVES, s1 = (w + 1) * NS / CS_WAVES;
+  const int r = r0 + cl, co = co0 + cl;
+  const bool vec = c.Cin % 4 == 0 && c.ldx % 4 == 0;  // 16-byte loads of whole 4-channel groups
+  const float* wrow = c.w + ((size_t)ph * c.Cout + (co < c.Cout ? co : 0)) * c.taps * c.Cin;
+
+  // step st: tap j = st / nch, this lane's channels cc .. cc + 7 with cc = (st % nch) * 32 + g * 8
+  auto load = [&](int st, float (&xv)[8], float (&wv)[8]) {
+    const int j = st / nch, cc = (st - j * nch) * 32 + g * 8;
+    const int in_row = r * c.s_in + j * c.d_in + c.off_in[ph];
+    const bool rok = r <= r_hi && in_row >= 0 && in_row < Tin, wok = co < c.Cout;
+    const float* xp = xb + (size_t)(rok ? in_row : 0) * c.ldx + cc;
+    const float* wp = wrow + (size_t)j * c.Cin + cc;
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      if (vec && cc + e + 3 < c.Cin) {
+        const float4 x4 = rok ? *(const float4*)(xp + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 w4 = wok ? *(const float4*)(wp + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+        xv[e] = x4.x; xv[e + 1] = x4.y; xv[e + 2] = x4.z; xv[e + 3] = x4.w;
+        wv[e] = w4.x; wv[e + 1] = w4.y; wv[e + 2] = w4.z; wv[e + 3] = w4.w;
+      } else {
+#pragma unroll
+        for (int u = e; u < e + 4; ++u) {
+          xv[u] = rok && cc + u < c.Cin ? xp[u] : 0.f;
+          wv[u] = wok && cc + u < c.Cin ? wp[u] : 0.f;
+        }
+      }
+    }
+  };
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](int st, const float (&xv)[8], const float (&wv)[8]) {
+    const int j = st / nch, cc = (st - j * nch) * 32 + g * 8;
+    const int in_row = r * c.s_in + j * c.d_in + c.off_in[ph];
+    const bool rok = r <= r_hi && in_row >= 0 && in_row < Tin;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int ci = cc + u;
+      float v = xv[u];
+      if (c.pre && rok && ci < c.Cin) v = pre_act(v, c.pre, c.slope, c.alpha ? c.alpha[ci] : 0.f, c.inv ? c.inv[ci] : 0.f);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u], v, acc, 0, 0, 0);
+    }
+  };
+  constexpr int D = 4;  // steps in flight
+  float xv[D][8], wv[D][8];
+#pragma unroll
+  for (int q = 0; q < D; ++q)
+    if (s0 + q < s1) load(s0 + q, xv[q], wv[q]);
+  for (int st = s0; st < s1; st += D) {
+#pragma unroll
+    for (int q = 0; q < D; ++q)
+      if (st + q < s1) {
+        mma(st + q, xv[q], wv[q]);
+        if (st + q + D < s1) load(st + q + D, xv[q], wv[q]);
+      }
+  }
+  red[w][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  __syncthreads();
+  if (tid >= 64) return;
+  float4 sum = red[0][lane];
+#pragma unroll
+  for (int x = 1; x < CS_WAVES; ++x) {
+    const float4 v = red[x][lane];
+    sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+  }
+  // the lane holds output row r and channels co0 + g * 4 + 0..3
+  const int cn = g * 4, ncols = min(16, c.Cout - co0);
+  if (r > r_hi || cn >= ncols) return;
+  const size_t orow = (size_t)c.out_off[b] + (size_t)(r * c.s_out + oo);
+  if (cn + 3 < ncols) conv_epilogue4<true>(c, orow, co0 + cn, sum);
+  else conv_epilogue_part<true>(c, orow, co0 + cn, ncols - cn, sum);
+}
+
 // f0 = |w . x + b| per frame (one wave per frame row, Linear(C -> 1) then abs)
 __global__ void __launch_bounds__(256) f0_head_kernel(const float* x, int C, const float* w, const float* b, float* f0, int rows) {
   const int lane = threadIdx.x & 63;
@@ -1536,9 +1624,16 @@ hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st) {
   // grids that would keep fewer than half the CUs busy: 32-row tiles with the taps and channels split over the waves
   const long tiles = (long)cdiv(max_rows, 64) * cdiv(c.Cout, 64) * c.n_items * c.n_phase;
   if (tiles < 128) {
-    // 32 output channels per workgroup while that grid fits the chip in one round (half the weight bytes each), else 64
+    // 16 x 16 tiles while those are at most two to a CU (whole calls of one 190-frame row 1,190 -> 1,137 us, of four 58-frame
+    // windows 1,338 -> 1,291; at up to four to a CU eight such windows go 1,977 -> 2,001, two 221-frame rows 1,967 ->
+    // 1,983), 32 output channels per workgroup while that grid fits the chip in one round (half the weight bytes each),
+    // else 64
     const long t32 = (long)cdiv(max_rows, 32) * cdiv(c.Cout, 32) * c.n_items * c.n_phase;
-    if (t32 <= 256) {
+    const long t16 = (long)cdiv(max_rows, 16) * cdiv(c.Cout, 16) * c.n_items * c.n_phase;
+      if (t16 <= 512) {
+      dim3 grid(cdiv(max_rows, 16), cdiv(c.Cout, 16), c.n_items * c.n_phase);
+      hipLaunchKernelGGL(conv_f32_split16_kernel, grid, dim3(64 * CS_WAVES), 0, st, c);
+    } else if (t32 <= 256) {
       dim3 grid(cdiv(max_rows, 32), cdiv(c.Cout, 32), c.n_items * c.n_phase);
       hipLaunchKernelGGL(conv_f32_split_kernel<1>, grid, dim3(64 * CS_WAVES), 0, st, c);
     } else {

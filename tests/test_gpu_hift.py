@@ -184,6 +184,27 @@ def test_window_calls_side_by_side(lens, S):
     assert e < 5e-3
 
 
+@pytest.mark.parametrize("lens", [[1], [2, 1], [15], [16], [17, 33], [34], [35], [190], [255], [256], [257]], ids=str)
+def test_small_fp32_convs(lens):
+    """Calls of up to 256 frames run the f0 predictor's convs on 16 x 16 tiles, of up to 34 conv_post (18 channels) and of
+    one or two frames most of the strict-fp32 decoder; on both sides of the tiles' edges and of the rule's.  The f0 bound
+    is five fp32 convs' rounding (K = 1536 sums, relative 6e-8 x sqrt(1536) = 2.3e-6 each), the decoder's the
+    reference's."""
+    W = init_hift(HiFTConfig(), seed=8)
+    g = torch.Generator().manual_seed(sum(lens))
+    mels = [torch.randn(1, 80, t, generator=g) * 2 - 5 for t in lens]
+    noise = [oh.hift_noise(9, [100 + i], t * 480) for i, t in enumerate(lens)]
+    h, gm = oh.HiFT(W), HiFTModel(W, HiFTConfig())
+    mel_tm, noise_tm = _packed(mels, noise)
+    srcs = [oh.source(h, m, torch.zeros(1, 1, 0), ri, nz) for m, (ri, nz) in zip(mels, noise)]
+    s_tm = torch.cat([s[0, 0] for s in srcs]).cuda()
+    sp, _, f0 = gm.forward_packed(lens, mel_tm, noise_tm, None, 0, source_override=s_tm, want_f0=True)
+    e0 = rel(f0.cpu(), torch.cat([h.f0_predictor(m)[0] for m in mels]))
+    e = rel(sp.cpu(), torch.cat([oh.decode(h, m, s)[0] for m, s in zip(mels, srcs)]))
+    print("small fp32 convs", lens, "f0 rel-L2", e0, "decoder rel-L2", e)
+    assert e0 < 1.2e-5 and e < 1e-4
+
+
 def test_hift_graphs_equal_eager():
     """Graph replays (one graph per row lengths and source-cache length) equal eager calls bit for bit, replay after
     replay with new inputs, eager work and synchronisations in between; a second key gets its own graph."""
