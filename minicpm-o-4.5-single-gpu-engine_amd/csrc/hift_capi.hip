@@ -449,8 +449,8 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
   float* Sb = B.S;
   const int scls[3] = {C_S0, C_S1, C_S2};
   // Window calls: a stage's three ResBlocks run side by side (one launch per conv of the three), and so do the three
-  // stages' source branches, which need nothing of the decoder, before it; each value is computed as below.  One
-  // 58-frame window: 62 conv launches -> 29.
+  // stages' source branches, which need nothing of the decoder, before it; each value is computed as below.  The 72
+  // ResBlock convs take 24 launches.
   const bool win = window_call(x, B);
   auto source_down = [&](int i, float* y) {
     const int r = i == 0 ? d.up_rates[2] * d.up_rates[1] : (i == 1 ? d.up_rates[2] : 1);
