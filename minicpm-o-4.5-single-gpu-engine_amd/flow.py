@@ -384,9 +384,10 @@ class FlowEncoder:
             if wr is not None:
                 self.pc.drop(wr)
             raise
-        # advance the lists: [cache, new]; the first stack as the first half of the trimmed tiled list.  All streams' new
-        # lists are held before any old one, and the call's own references to its new slots, are dropped
-        old1, old2, oldc, new_c = [new1], [new2], [wr], []
+        # advance the lists: [cache, new]; the first stack as the first half of the trimmed tiled list.  Every window's new
+        # lists are held before any old one, and the call's own references to its new slots, are dropped.  A state named by
+        # several windows ends with its last window's lists: each later window drops what the one before it held
+        old1, old2, oldc, now1, now2, now_c = [new1], [new2], [wr], [], [], []
         for r, st in enumerate(states):
             c1 = kv1[kv1_off[r]:kv1_off[r] + L1[r]]
             c2 = kv2[kv2_off[r]:kv2_off[r] + L2[r]]
@@ -401,10 +402,12 @@ class FlowEncoder:
                 st.k1 = p1[: p1.size // 2].astype(np.int32)
                 st.k2 = _trim(c2, st.keep).astype(np.int32)
                 st.cnn = int(wr[r])
-                new_c.append(st.cnn)
-        self.p1.hold(np.concatenate([st.k1 for st in states]))
-        self.p2.hold(np.concatenate([st.k2 for st in states]))
-        self.pc.hold(new_c)
+                now_c.append(st.cnn)
+            now1.append(st.k1)
+            now2.append(st.k2)
+        self.p1.hold(np.concatenate(now1))
+        self.p2.hold(np.concatenate(now2))
+        self.pc.hold(now_c)
         self.p1.drop(np.concatenate(old1))
         self.p2.drop(np.concatenate(old2))
         self.pc.drop(np.concatenate(oldc))

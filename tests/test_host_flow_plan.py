@@ -174,3 +174,29 @@ def test_ref_pool_counts_duplicates():
     p.drop([])
     with pytest.raises(RuntimeError):
         p.drop([ids[1]])
+
+
+@pytest.mark.parametrize("lasts", [[False, False], [False, False, False], [False, True], [True, False], [True, True]], ids=str)
+def test_one_state_in_several_windows(enc, lasts):
+    """A state may be named by several windows of a call: every window reads the lists it had before the call, the state
+    ends with its last window's, and the pools hold just that."""
+    rng = np.random.default_rng(2)
+    [st], _, _, _ = enc.setup([rng.integers(0, CFG.vocab, 17).tolist()])
+    k1, k2 = st.k1.copy(), st.k2.copy()
+    other = enc.new_state(10)
+    enc.encode([st, other, *[st] * (len(lasts) - 1)], [rng.integers(0, CFG.vocab, 20).tolist() for _ in range(len(lasts) + 1)],
+               [lasts[0], True, *lasts[1:]])
+    if lasts[-1]:
+        assert st.k1.size == 0 and st.k2.size == 0 and st.cnn == enc.zero_cnn
+    else:
+        assert np.array_equal(st.k1, np.concatenate([k1, enc_new(enc, 1)[-17:]]))
+        assert np.array_equal(st.k2, np.concatenate([k2, enc_new(enc, 2)[-34:]]))
+        assert st.cnn == lib_calls(enc)[-1]["cnn_wr"][-1]
+    assert enc.in_use() == (st.k1.size, st.k2.size, int(st.cnn != enc.zero_cnn))
+    for pool, ids in ((enc.p1, st.k1), (enc.p2, st.k2), (enc.pc, [st.cnn] if st.cnn else [])):
+        want = np.zeros_like(pool.ref)
+        want[enc.pc.reserved] = pool.ref[enc.pc.reserved] if pool is enc.pc else 0
+        want[ids] = 1
+        assert np.array_equal(pool.ref, want)
+    enc.release(st)
+    assert enc.in_use() == (0, 0, 0)
