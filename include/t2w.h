@@ -332,7 +332,9 @@ typedef struct {
 int t2w_hift_create(const t2w_hift_dims* dims, const t2w_hift_weights* w, t2w_hift** out);
 void t2w_hift_destroy(t2w_hift* h);
 /* Plan of a call over n_items rows with frames[i] mel frames (host array): ints for t2w_hift_plan to fill, which the
- * caller copies to device memory; workspace bytes. */
+ * caller copies to device memory; workspace bytes.  A short call (bf16 decoder, up to about 318 frames) asks for room to
+ * run a stage's ResBlocks side by side; given a workspace sized for longer rows that is smaller than this, it runs them
+ * one after another instead (the same result up to the order of fp32 sums). */
 int t2w_hift_plan_ints(int n_items);
 int t2w_hift_plan(const t2w_hift* h, int n_items, const int* frames, int* plan_host);
 size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n_items, const int* frames);

@@ -92,7 +92,9 @@ bool window_sized(const t2w_hift* h, const Lens& L, int n) {
   return true;
 }
 
-size_t carve(const t2w_hift* h, const Lens& L, int n, char* base, Bufs* b) {
+// The side-by-side buffers (window) come last, so a workspace without them still holds the rest.  That rest never
+// shrinks when a row gets longer or a row is added; with them it does (only short calls have them).
+size_t carve(const t2w_hift* h, const Lens& L, bool window, char* base, Bufs* b) {
   const t2w_hift_dims& d = h->d;
   size_t big = 0;
   big = std::max(big, (size_t)L.tot[C_T] * d.base);
@@ -117,7 +119,7 @@ size_t carve(const t2w_hift* h, const Lens& L, int n, char* base, Bufs* b) {
   const int scls[3] = {C_S0, C_S1, C_S2};
   for (int i = 0; i < 3; ++i) {
     t.wz[i] = t.wt[i] = t.ws[i] = t.wst[i] = nullptr;
-    if (!window_sized(h, L, n)) continue;
+    if (!window) continue;
     t.wz[i] = take(big);
     t.wt[i] = take(big);
     t.ws[i] = take((size_t)L.tot[scls[i]] * h->chans[i + 1]);
@@ -376,7 +378,8 @@ int t2w_hift_plan(const t2w_hift* h, int n, const int* frames, int* plan) {
 
 size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n, const int* frames) {
   if (!h || n <= 0) return 0;
-  return carve(h, lens_of(h->d, n, frames), n, nullptr, nullptr);
+  const Lens L = lens_of(h->d, n, frames);
+  return carve(h, L, window_sized(h, L, n), nullptr, nullptr);
 }
 
 int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* plan_dev, const float* mel, const float* noise,
@@ -388,9 +391,12 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
   for (int i = 0; i < n; ++i)
     if (S > class_len(d, C_SMP, frames[i])) return t2w::set_error("source cache longer than a row", hipSuccess);
   if (S > 0 && !cache_source) return t2w::set_error("missing source cache", hipSuccess);
-  if (workspace_bytes < carve(h, x.L, n, nullptr, nullptr)) return t2w::set_error("hift workspace too small", hipSuccess);
+  if (workspace_bytes < carve(h, x.L, false, nullptr, nullptr)) return t2w::set_error("hift workspace too small", hipSuccess);
+  // a workspace sized for longer rows may not hold the side-by-side buffers of a short call: its ResBlocks then run one
+  // after another
+  const bool room = window_sized(h, x.L, n) && workspace_bytes >= carve(h, x.L, true, nullptr, nullptr);
   Bufs B;
-  carve(h, x.L, n, (char*)workspace, &B);
+  carve(h, x.L, room, (char*)workspace, &B);
   const t2w_hift_weights& w = h->w;
   const int harm = d.harmonics + 1, nsrc = d.n_fft + 2;
 

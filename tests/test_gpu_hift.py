@@ -8,10 +8,13 @@ to end is held to 5e-4 (it measures ~4e-5: its f0 matches the oracle's to 2e-6, 
 the bf16 decoders to the reference's reduced-precision HiFT bound of 1e-2 (``tests/engine/test_hift_tf32.py:227``).
 """
 
+import ctypes
+
 import pytest
 import torch
 
 import t2w_amd  # noqa: F401
+from t2w_amd import _lib
 from t2w_amd.config import HiFTConfig
 from t2w_amd.hift import HiFTModel
 from t2w_amd.weights import init_hift
@@ -182,6 +185,32 @@ def test_window_calls_side_by_side(lens, S):
     e = rel(outs[0][0].cpu(), outs[1][0].cpu())
     print("window call", lens, S, "rel-L2", e)
     assert e < 5e-3
+
+
+@pytest.mark.parametrize("longer,lens", [([319], [318]), ([400], [300]), ([165, 60], [74, 60]), ([60] * 7, [60] * 5)], ids=str)
+def test_workspace_of_longer_rows(longer, lens):
+    """A workspace sized for one call serves every call whose rows are no longer and no more, also where the shorter call
+    would ask for more room (its ResBlocks side by side): the same waveform up to the order of fp32 sums (bound as in
+    test_window_calls_side_by_side), the same source, and nothing written past the workspace's end."""
+    L, hm = _lib.lib(), HiFTModel(init_hift(HiFTConfig(), seed=6), HiFTConfig(), decode_bf16=True)
+    need = lambda fr: int(L.t2w_hift_workspace_bytes(hm.handle, len(fr), (ctypes.c_int * len(fr))(*fr)))  # noqa: E731
+    g = torch.Generator().manual_seed(sum(lens))
+    mel = (torch.randn(sum(lens), 80, generator=g) * 2 - 5).cuda()
+    noise = torch.randn(sum(lens) * 480, 9, generator=g).cuda()
+    want, wsrc, _ = hm.forward_packed(lens, mel, noise, None, 0)
+    size = need(longer)
+    ws = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    n, fr = len(lens), (ctypes.c_int * len(lens))(*lens)
+    plan = (ctypes.c_int * L.t2w_hift_plan_ints(n))()
+    _lib.check(L.t2w_hift_plan(hm.handle, n, fr, plan), "plan")
+    plan_dev = torch.tensor(list(plan), dtype=torch.int32).cuda()
+    speech, source = torch.empty_like(want), torch.empty_like(wsrc)
+    _lib.check(L.t2w_hift_forward(hm.handle, n, fr, plan_dev.data_ptr(), mel.data_ptr(), noise.data_ptr(), None, 0, None, None,
+                                  speech.data_ptr(), source.data_ptr(), None, ws.data_ptr(), size, 1, _lib.stream_handle()), "forward")
+    torch.cuda.synchronize()
+    print("workspace", size, "own", need(lens))
+    assert torch.equal(source, wsrc) and rel(speech, want) < 5e-3
+    assert bool((ws[size:] == 0x5A).all())
 
 
 @pytest.mark.parametrize("lens", [[1], [2, 1], [15], [16], [17, 33], [34], [35], [190], [255], [256], [257]], ids=str)
