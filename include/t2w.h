@@ -338,6 +338,8 @@ void t2w_hift_destroy(t2w_hift* h);
 int t2w_hift_plan_ints(int n_items);
 int t2w_hift_plan(const t2w_hift* h, int n_items, const int* frames, int* plan_host);
 size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n_items, const int* frames);
+/* t2w_hift_workspace_bytes for calls of one decode_bf16 mode (0 and 3 never run ResBlocks side by side and ask for less) */
+size_t t2w_hift_workspace_bytes_for(const t2w_hift* h, int n_items, const int* frames, int decode_bf16);
 /* hift_forward_noise for rows of different lengths, time-major and packed: mel [sum T, mel]; noise [sum 480 T, harmonics
  * + 1]; cache_source [n_items, S] replaces each row's first S source samples; speech / source out [sum 480 T].
  * f0_override / source_override (optional, device): use these instead of the f0 predictor / the NSF source. f0_out

@@ -122,6 +122,7 @@ _SIGS = {
     "t2w_hift_plan_ints": (I, [I]),
     "t2w_hift_plan": (I, [P, I, P, P]),
     "t2w_hift_workspace_bytes": (C.c_size_t, [P, I, P]),
+    "t2w_hift_workspace_bytes_for": (C.c_size_t, [P, I, P, I]),
     "t2w_hift_forward": (I, [P, I, P, P, P, P, P, I, P, P, P, P, P, P, C.c_size_t, I, P]),
     "t2w_flow_create": (I, [C.POINTER(FlowDims), C.POINTER(P)]),
     "t2w_flow_set_layer": (I, [P, I, C.POINTER(FlowLayer)]),

@@ -84,8 +84,10 @@ struct Bufs {
   float *wz[3], *wt[3], *ws[3], *wst[3];
 };
 
-// Calls small enough that the window kernel takes every stage's ResBlock convs: their ResBlocks run side by side
-bool window_sized(const t2w_hift* h, const Lens& L, int n) {
+// Calls small enough that the window kernel takes every stage's ResBlock convs: their ResBlocks run side by side.  Only
+// the bf16 decoder does that, and not where every dilation is one fused kernel (decode_bf16 0 and 3).
+bool window_sized(const t2w_hift* h, const Lens& L, int n, int decode_bf16) {
+  if (decode_bf16 == 0 || decode_bf16 == 3) return false;
   const int cls[3] = {C_S0, C_S1, C_S2};
   for (int i = 0; i < 3; ++i)
     if ((long)((L.mx[cls[i]] + 2 + 127) / 128) * ((h->chans[i + 1] + 63) / 64) * n >= CONV_WINDOW_BATCH_TILES) return false;
@@ -266,7 +268,7 @@ int window_blocks(const Ctx& x, const WindowBlock (&wb)[3], const char* what) {
 
 // whether every ResBlock conv of the call fits the window kernel (bf16 weights, spans, sizes)
 bool window_call(const Ctx& x, const Bufs& B) {
-  if (!x.bf16 || x.fuse == 2 || !B.wz[0]) return false;
+  if (!B.wz[0]) return false;  // not a window call, or a workspace without their buffers
   const t2w_hift_dims& d = x.h->d;
   const int scls[3] = {C_S0, C_S1, C_S2};
   for (int i = 0; i < 3; ++i)
@@ -376,10 +378,12 @@ int t2w_hift_plan(const t2w_hift* h, int n, const int* frames, int* plan) {
   return 0;
 }
 
-size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n, const int* frames) {
+size_t t2w_hift_workspace_bytes(const t2w_hift* h, int n, const int* frames) { return t2w_hift_workspace_bytes_for(h, n, frames, 1); }
+
+size_t t2w_hift_workspace_bytes_for(const t2w_hift* h, int n, const int* frames, int decode_bf16) {
   if (!h || n <= 0) return 0;
   const Lens L = lens_of(h->d, n, frames);
-  return carve(h, L, window_sized(h, L, n), nullptr, nullptr);
+  return carve(h, L, window_sized(h, L, n, decode_bf16), nullptr, nullptr);
 }
 
 int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* plan_dev, const float* mel, const float* noise,
@@ -394,7 +398,7 @@ int t2w_hift_forward(const t2w_hift* h, int n, const int* frames, const int* pla
   if (workspace_bytes < carve(h, x.L, false, nullptr, nullptr)) return t2w::set_error("hift workspace too small", hipSuccess);
   // a workspace sized for longer rows may not hold the side-by-side buffers of a short call: its ResBlocks then run one
   // after another
-  const bool room = window_sized(h, x.L, n) && workspace_bytes >= carve(h, x.L, true, nullptr, nullptr);
+  const bool room = window_sized(h, x.L, n, decode_bf16) && workspace_bytes >= carve(h, x.L, true, nullptr, nullptr);
   Bufs B;
   carve(h, x.L, room, (char*)workspace, &B);
   const t2w_hift_weights& w = h->w;

@@ -154,7 +154,7 @@ class HiFTModel:
 
     def _workspace(self, frames: list[int]) -> torch.Tensor:
         fr = (C.c_int * len(frames))(*frames)
-        need = _lib.lib().t2w_hift_workspace_bytes(self.handle, len(frames), fr)
+        need = _lib.lib().t2w_hift_workspace_bytes_for(self.handle, len(frames), fr, self._mode)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device=self.device)
         return self._ws
@@ -206,7 +206,7 @@ class HiFTModel:
                  "mel": torch.zeros(sum(frames), self.cfg.mel, device=dev), "noise": torch.zeros(ns, self.dim, device=dev),
                  "cs": torch.zeros(n, S, device=dev) if S > 0 else None,
                  "speech": torch.empty(ns, device=dev), "source": torch.empty(ns, device=dev),
-                 "ws": torch.empty(L.t2w_hift_workspace_bytes(self.handle, n, fr), dtype=torch.uint8, device=dev)}
+                 "ws": torch.empty(L.t2w_hift_workspace_bytes_for(self.handle, n, fr, self._mode), dtype=torch.uint8, device=dev)}
             cap = self._capture_stream()  # capture needs a non-default stream; replays go on the caller's
             cap.wait_stream(torch.cuda.current_stream())
             cst = cap.cuda_stream

@@ -213,6 +213,18 @@ def test_workspace_of_longer_rows(longer, lens):
     assert bool((ws[size:] == 0x5A).all())
 
 
+@pytest.mark.parametrize("kw,mode", [({}, 0), ({"decode_bf16": True}, 1), ({"decode_bf16": True, "resblock_fusion": "off"}, 2),
+                                     ({"decode_bf16": True, "resblock_fusion": "on"}, 3)], ids=["fp32", "auto", "off", "on"])
+def test_workspace_holds_what_the_mode_runs(kw, mode):
+    """Only the modes that run a short call's ResBlocks side by side hold the buffers for it."""
+    L, hm = _lib.lib(), HiFTModel(init_hift(HiFTConfig(), seed=6), HiFTConfig(), **kw)
+    need = lambda t, m: int(L.t2w_hift_workspace_bytes_for(hm.handle, 1, (ctypes.c_int * 1)(t), m))  # noqa: E731
+    assert need(58, 0) == need(58, 3) < need(58, 1) == need(58, 2) == L.t2w_hift_workspace_bytes(hm.handle, 1, (ctypes.c_int * 1)(58))
+    assert need(400, 0) == need(400, 1) == need(400, 2) == need(400, 3)
+    out = hm.forward_packed([58], torch.zeros(58, 80, device="cuda"), torch.zeros(58 * 480, 9, device="cuda"), None, 0)[0]
+    assert hm._ws.numel() == need(58, mode) and bool(torch.isfinite(out).all())
+
+
 @pytest.mark.parametrize("lens", [[1], [2, 1], [15], [16], [17, 33], [34], [35], [190], [255], [256], [257]], ids=str)
 def test_small_fp32_convs(lens):
     """Calls of up to 256 frames run the f0 predictor's convs on 16 x 16 tiles, of up to 34 conv_post (18 channels) and of
