@@ -264,6 +264,22 @@ int t2w_gemm_bf16(const void* A, int lda, const int* a_src, const void* W, const
  * K % 64 == 0, lda % 8 == 0 (taps mode: lda % 64 == 0). */
 int t2w_gemm_bf16_tile(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate,
                        void* C, int ldc, int M, int N, int K, int epi, int tile, void* stream);
+/* One GEMM on a named ring tile with any epilogue the ring has, bf16 or (w_scale non-null) fp8 as t2w_gemm_fp8.
+ * tile: 0 64x64, 1 128x64, 2 128x128, 3 192x128, 4 256x128.  epi: as t2w_gemm_bf16, and
+ *   4  fp8 GELU, MX fp8 codes to C (rows ldc) and block scales to c_scale (rows N / 32)
+ *   5  qkv (N = 3 H, H % 64 == 0; not tile 1, fp8 not tile 3; N a multiple of the tile's columns): per-head LayerNorm of
+ *      q and k, q to its row of q_out [M, H], k and v to slot slots[m] of the pools (C unused)
+ *   6  K split `splits` ways (tiles 0 to 2, bf16): split z's plain fp32 sums to C + z * M * ldc (bias unused)
+ * What the tile or epilogue does not take is refused before any launch. */
+typedef struct {
+  const void* A; int lda; const int* a_src; const void* a_scale; int a_sld;
+  const void* W; const float* w_scale; const float* bias; const float* gate;
+  void* C; int ldc; void* c_scale;
+  int M, N, K, epi, tile, splits;
+  void* q_out; void* k_pool; void* v_pool; const int* slots;
+  const float* qn_w; const float* qn_b; const float* kn_w; const float* kn_b; float eps_qk; int H;
+} t2w_ring_args;
+int t2w_gemm_ring(const t2w_ring_args* a, void* stream);
 /* t2w_gemm_bf16 with a workspace for split-K partials (256-byte aligned; up to splits x M x N fp32): a call that
  * neither the small-row kernel nor the ring tiles take (16-bit output rows that are not 16-byte aligned) and whose tile
  * grid would leave most CUs idle splits K over ~512 waves and reduces the partials in a fixed order. */

@@ -50,6 +50,12 @@ class DitBlockFp8(C.Structure):
                                  "fc2_w8", "fc2_ws")]
 
 
+class RingArgs(C.Structure):
+    _fields_ = [("A", P), ("lda", I), ("a_src", P), ("a_scale", P), ("a_sld", I), ("W", P), ("w_scale", P), ("bias", P), ("gate", P),
+                ("C", P), ("ldc", I), ("c_scale", P)] + [(n, I) for n in ("M", "N", "K", "epi", "tile", "splits")] + \
+               [(n, P) for n in ("q_out", "k_pool", "v_pool", "slots", "qn_w", "qn_b", "kn_w", "kn_b")] + [("eps_qk", F), ("H", I)]
+
+
 class HiftDims(C.Structure):
     _fields_ = [(n, I) for n in ("mel", "base", "n_up", "harmonics", "f0_channels", "f0_layers", "sr", "n_fft", "hop")] + \
                [(n, I * 3) for n in ("up_rates", "up_kernels", "res_kernels", "res_dilations", "src_kernels")] + \
@@ -111,6 +117,7 @@ _SIGS = {
     "t2w_gemm_bf16": (I, [P, I, P, P, P, P, P, I, I, I, I, I, P]),
     "t2w_gemm_bf16_tile": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, P]),
     "t2w_gemm_bf16_ws": (I, [P, I, P, P, P, P, P, I, I, I, I, I, P, C.c_size_t, P]),
+    "t2w_gemm_ring": (I, [C.POINTER(RingArgs), P]),
     "t2w_quant_mx8": (I, [P, I, I, I, P, I, P, P]),
     "t2w_dit_set_block_fp8": (I, [P, I, P]),
     "t2w_gemm_fp8": (I, [P, I, P, P, I, P, P, P, P, P, I, I, I, I, I, P]),

@@ -617,6 +617,26 @@ int t2w_gemm_bf16_ws(const void* A, int lda, const int* a_src, const void* W, co
   return 0;
 }
 
+int t2w_gemm_ring(const t2w_ring_args* a, void* stream) {
+  if (!a || !a->A || !a->W || a->lda <= 0) return fail("ring gemm: null operand");
+  if (a->a_src && a->K % a->lda) return fail("ring gemm: taps mode needs K a multiple of lda");
+  const bool qkv = a->epi == EPI_QKV, part = a->epi == EPI_PART;
+  if (qkv ? !a->q_out || !a->k_pool || !a->v_pool || !a->slots || !a->qn_w || !a->qn_b || !a->kn_w || !a->kn_b : !a->C)
+    return fail("ring gemm: null output");
+  if ((!part && !a->bias) || (a->epi == EPI_RESID_F16 && !a->gate) || (a->w_scale && !a->a_scale)) return fail("ring gemm: null bias, gate or scale");
+  GemmArgs g = gemm_args(a->A, a->lda, a->a_src, a->W, a->bias, a->gate, a->C, a->ldc, a->M, a->N, a->K);
+  g.a_scale = (const uint8_t*)a->a_scale;
+  g.a_sld = a->a_sld;
+  g.w_scale = a->w_scale;
+  g.c_scale = (uint8_t*)a->c_scale;
+  g.c_sld = a->N / 32;
+  g.qk = QkvOut{(bf16_t*)a->q_out, (bf16_t*)a->k_pool, (bf16_t*)a->v_pool, a->slots, a->qn_w, a->qn_b, a->kn_w, a->kn_b, a->eps_qk, a->H};
+  g.splits = a->splits;
+  g.c_split = (size_t)a->M * a->ldc;
+  T2W_CHECK(gemm_ring(g, a->epi, a->tile, (hipStream_t)stream), "ring gemm");
+  return 0;
+}
+
 int t2w_quant_mx8(const void* x, int ldx, int M, int K, void* q, int ldq, void* scales, void* stream) {
   if (K % 32 || ldx % 8 || ldq % 8) return fail("quant_mx8: K % 32, ldx % 8 and ldq % 8 must be 0");
   T2W_CHECK(quant_mx8((const bf16_t*)x, ldx, M, K, (uint8_t*)q, ldq, (uint8_t*)scales, (hipStream_t)stream), "quant_mx8");

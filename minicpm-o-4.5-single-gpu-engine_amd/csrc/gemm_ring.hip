@@ -365,7 +365,7 @@ RingPlan ring_plan(int M, int N, int K, int max_splits, bool qkv, bool fp8) {
   const int ke = fp8 ? 128 : 64;
   if (K % ke) return p;
   for (int c = 0; c < 5; ++c) {
-    if (qkv && (c == 1 || (fp8 && c == 3))) continue;
+    if (qkv && (c == 1 || (fp8 && c == 3) || N % RING[c].bn)) continue;
     for (int S = 1; S <= (c < 3 ? max_splits : 1) && S <= K / ke; ++S) {
       const long ns = ring_ns(c, M, N, K / ke, S);
       if (ns >= 0 && (best < 0 || ns < best)) best = ns, p.cfg = c, p.splits = S;
@@ -399,7 +399,9 @@ bool gemm_ring_fits(const GemmArgs& g, int epi) {
 }
 
 hipError_t gemm_ring(const GemmArgs& g, int epi, int cfg, hipStream_t st) {
-  if (!gemm_ring_fits(g, epi)) return hipErrorInvalidValue;
+  if (cfg < 0 || cfg >= 5 || !gemm_ring_fits(g, epi)) return hipErrorInvalidValue;
+  // the qkv store has no column guard: columns past N would be written as one more head of v
+  if (epi == EPI_QKV && g.N % RING[cfg].bn) return hipErrorInvalidValue;
   const int e = epi * 2 + (g.a_src ? 1 : 0);
   if (g.w_scale) {
     switch (e) {
