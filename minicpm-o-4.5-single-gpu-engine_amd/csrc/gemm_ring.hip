@@ -377,6 +377,9 @@ RingPlan ring_plan(int M, int N, int K, int max_splits, bool qkv, bool fp8) {
 bool gemm_ring_fits(const GemmArgs& g, int epi) {
   const bool taps = g.a_src != nullptr;
   if (g.M <= 0 || g.N <= 0 || g.K <= 0 || (((size_t)g.A | (size_t)g.B) & 15)) return false;  // 16-byte copies
+  // both operands are addressed by 32-bit byte offsets (taps: frame rows up to M + 65536)
+  const size_t es = g.w_scale ? 1 : 2;
+  if (((size_t)g.M + 65536) * g.lda * es >= ((size_t)1 << 32) || (size_t)g.N * g.ldb * es >= ((size_t)1 << 32)) return false;
   if (g.w_scale) {
     // codes and scale dwords (4 blocks of 32 K values); taps: the scale rows run on across frames like the codes
     if (g.K % 128 || g.lda % 16 || g.ldb % 16 || g.a_sld % 4 || ((size_t)g.a_scale & 3) || (taps && g.a_sld * 32 != g.lda)) return false;

@@ -48,3 +48,10 @@ def ring_refuses(**kw):
 def test_ring_qkv_needs_whole_tiles(tile):
     """A 128-column tile over 3 H columns that are not a multiple of 128 would store the overhang as a head of v."""
     ring_refuses(epi=5, tile=tile, H=960, N=2880, K=960, lda=960)
+
+
+@pytest.mark.parametrize("kw", [{"M": (1 << 21) - 65536}, {"M": (1 << 31) - 1}, {"N": 1 << 21}, {"M": (1 << 21) - 65536, "epi": 6, "splits": 2}], ids=str)
+def test_ring_refuses_operands_beyond_32_bit_offsets(kw):
+    """The ring's copies name their rows by 32-bit byte offsets: operands of 4 GiB are refused by the ring itself, whoever
+    calls it."""
+    ring_refuses(tile=0, **kw)
