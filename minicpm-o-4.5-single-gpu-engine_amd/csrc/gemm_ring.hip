@@ -92,12 +92,11 @@ struct Ring {
   // Stage kt into the ring slot at LDS byte address `slot`.  The copies are inline assembly so that the compiler does
   // not count them: it would wait for every load in flight before the first fragment read of a loop, which is what
   // the ring is there to avoid; wait_vm and the barrier in stage() order them instead.  They have no output registers.
-  // (M0 is not otherwise used here.)
   __device__ __forceinline__ void dma(uint32_t lds, uint32_t off, const void* base) const {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
   }
   __device__ __forceinline__ void dma4(uint32_t lds, uint32_t off, const void* base) const {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
   }
   __device__ __forceinline__ void issue(uint32_t slot, int kt) const {
     const uint32_t koff = (uint32_t)kt * (BK * 2);  // taps: a row's frames follow each other, so K runs on across them
