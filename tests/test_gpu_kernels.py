@@ -139,11 +139,14 @@ def test_gemm_208_rows_equal_256(dev, M, N, epi):
         assert torch.equal(outs[0], outs[1]), (taps, epi)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 1024, 1024), (37, 3072, 1024), (100, 1024, 2048), (100, 80, 1024), (300, 2048, 1024), (600, 1024, 320)])
-@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 1024), (37, 3072, 1024), (100, 1024, 2048), (100, 80, 1024), (300, 2048, 1024), (600, 1024, 320),
+                                   (1, 1001, 1024), (37, 333, 128), (100, 77, 2048), (129, 65, 192), (300, 1001, 1024), (600, 1003, 320),
+                                   (1000, 130, 3072)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3, 7])
 def test_gemm_splitk(dev, M, N, K, epi):
-    """Calls with few rows split K over many waves (partials in the caller's workspace, fixed-order reduction):
-    parity with fp32 and bit-identical repeats."""
+    """Calls with a workspace for split-K partials: parity with fp32 and bit-identical repeats.  Rows of 16-byte multiples
+    take the small-row kernel or the ring tiles; the others split K over many waves (16 or 32 bit outputs, two to 48 K
+    steps, edges of its 64 columns and 128 rows), which without the workspace a 16-bit output is refused."""
     g = torch.Generator(device=dev).manual_seed(M + N + K + 5 * epi)
     A = torch.randn(M, K, device=dev, generator=g).bfloat16()
     W = (torch.randn(N, K, device=dev, generator=g) / K ** 0.5).bfloat16()
@@ -161,13 +164,18 @@ def test_gemm_splitk(dev, M, N, K, epi):
             out = torch.randn(M, N, device=dev, generator=torch.Generator(device=dev).manual_seed(9)).half()
             h0 = out.float()
         else:
-            out = torch.zeros(M, N, device=dev)
+            out = torch.zeros(M, N, device=dev, dtype=torch.float16 if epi == 7 else torch.float32)
+        if N % 4 and epi != 3:  # no other kernel takes these rows
+            with pytest.raises(RuntimeError, match="invalid argument"):
+                _gemm(A, W, bias, out, epi, gate=gate if epi == 2 else None)
         _gemm(A, W, bias, out, epi, gate=gate if epi == 2 else None, ws=ws)
         outs.append(out)
     if epi in (0, 1):
         assert rel(outs[0].float(), ref) < 6e-3
     elif epi == 2:
         assert rel(outs[0].float(), h0 + gate * ref) < 1e-3
+    elif epi == 7:
+        assert rel(outs[0].float(), ref) < 1e-3
     else:
         assert rel(outs[0], ref) < 1e-5
     assert torch.equal(outs[0], outs[1])
@@ -178,8 +186,8 @@ def test_gemm_splitk(dev, M, N, K, epi):
                                    (4200, 1000, 256), (6145, 1024, 192)])
 @pytest.mark.parametrize("epi", [0, 1, 2, 3, 7])
 def test_gemm_ring(dev, M, N, K, epi):
-    """The ring-buffered tiles (64x64 to 256x128 by shape) at the edges of tiles, of the ring (K of one to eight
-    stages) and of the output columns; dense and, where the epilogue has it, taps (rows of K / 64 64-value frames),
+    """The ring-buffered tiles (64x64 to 256x128 by shape) at the edges of tiles and of the output columns, K of one to 32
+    stages (every tile's refilled ring: test_gemm_ring_tiles); dense and, where the epilogue has it, taps (rows of K / 64 64-value frames),
     which read the same values and so give the same bits.  Bounds: one bf16 rounding is at most 2^-9 of a value, one
     fp16 rounding 2^-12, fp32 sums of up to 2048 products stay within 1e-5."""
     g = torch.Generator(device=dev).manual_seed(M + N + K + epi)
@@ -203,21 +211,152 @@ def test_gemm_ring(dev, M, N, K, epi):
     assert torch.equal(outs[0], outs[-1])
 
 
-def test_gemm_splitk_taps(dev):
-    """Split-K in taps mode (a streaming chunk's conv GEMM) equals the tile kernel's result for the same call."""
-    H, lens = 512, [50, 50]
+def _ring(tile, epi, A, W, M, N, K, bias, out=None, **kw):
+    """One t2w_gemm_ring call; keywords are further argument fields (tensors by their address)."""
+    a = _lib.RingArgs(A=A.data_ptr(), lda=K, W=W.data_ptr(), bias=bias.data_ptr(), C=_lib.ptr(out), ldc=N, M=M, N=N, K=K, epi=epi, tile=tile, splits=1,
+                      eps_qk=1e-6)
+    for k, v in kw.items():
+        setattr(a, k, v.data_ptr() if isinstance(v, torch.Tensor) else v)
+    _lib.check(_lib.lib().t2w_gemm_ring(C.byref(a), _lib.stream_handle()), "ring gemm")
+    torch.cuda.synchronize()
+
+
+RING_SHAPE = [(64, 64), (128, 64), (128, 128), (192, 128), (256, 128)]
+
+
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("tile", range(5))
+def test_gemm_ring_tiles(dev, tile, stages):
+    """Every ring tile and epilogue with K of one stage to more than four rounds of its ring (odd and even counts of
+    refilled stages), three row tiles with a remainder and one and a half column tiles: the bits of the two-buffer tile
+    kernel, which sums K in the same order, dense and taps."""
+    L, (bm, bn) = _lib.lib(), RING_SHAPE[tile]
+    M, N, K = 2 * bm + 37, bn + bn // 2 + 8, 64 * stages
+    g = torch.Generator(device=dev).manual_seed(100 * tile + stages)
+    frames = torch.randn(M + stages - 1, 64, device=dev, generator=g).bfloat16()
+    A = torch.cat([frames[j:j + M] for j in range(stages)], 1).contiguous()
+    src = torch.arange(M, dtype=torch.int32, device=dev)
+    W = (torch.randn(N, K, device=dev, generator=g) / K ** 0.5).bfloat16()
+    bias, gate = torch.randn(N, device=dev, generator=g), torch.randn(N, device=dev, generator=g)
+    for epi, dt in ((0, torch.bfloat16), (1, torch.bfloat16), (2, torch.float16), (3, torch.float32), (7, torch.float16)):
+        h0 = torch.randn(M, N, device=dev, generator=g).to(dt)
+        want = h0.clone()
+        _lib.check(L.t2w_gemm_bf16_tile(A.data_ptr(), K, None, W.data_ptr(), bias.data_ptr(), gate.data_ptr(), want.data_ptr(), N, M, N, K, epi, 0,
+                                        _lib.stream_handle()), "gemm tile")
+        for taps in (False, True) if epi in (0, 2, 3) else (False,):
+            out = h0.clone()
+            _ring(tile, epi, frames if taps else A, W, M, N, K, bias, out, gate=gate, **({"a_src": src, "lda": 64} if taps else {}))
+            assert torch.equal(out, want), (epi, taps)
+
+
+@pytest.mark.parametrize("stages,splits", [(1, 1), (2, 2), (4, 4), (5, 2), (7, 3), (11, 4), (16, 4), (32, 3), (48, 4)])
+@pytest.mark.parametrize("tile", range(3))
+def test_gemm_ring_part(dev, tile, stages, splits):
+    """EPI_PART: split z's plain sums over K stages z KT / S .. (z + 1) KT / S - 1, slices of unequal length among them,
+    dense and taps: the bits of the fp32 epilogue on each slice alone with a zero bias."""
+    bm, bn = RING_SHAPE[tile]
+    M, N, K = 2 * bm + 37, bn + bn // 2 + 8, 64 * stages
+    g = torch.Generator(device=dev).manual_seed(100 * tile + stages)
+    frames = torch.randn(M + stages - 1, 64, device=dev, generator=g).bfloat16()
+    A = torch.cat([frames[j:j + M] for j in range(stages)], 1).contiguous()
+    W = (torch.randn(N, K, device=dev, generator=g) / K ** 0.5).bfloat16()
+    zero = torch.zeros(N, device=dev)
+    want = torch.empty(splits, M, N, device=dev)
+    for z in range(splits):
+        k0, k1 = 64 * (z * stages // splits), 64 * ((z + 1) * stages // splits)
+        _ring(tile, 3, A[:, k0:k1].contiguous(), W[:, k0:k1].contiguous(), M, N, k1 - k0, zero, want[z])
+    for kw in ({}, {"a_src": torch.arange(M, dtype=torch.int32, device=dev), "lda": 64}):
+        out = torch.full((splits, M, N), 7.0, device=dev)
+        _ring(tile, 6, frames if kw else A, W, M, N, K, zero, out, splits=splits, **kw)
+        assert torch.equal(out, want)
+    assert rel(want.double().sum(0), A.double() @ W.double().t()) < 1e-5
+
+
+def _qkv_check(dev, run, pre, M, H, g):
+    """run(q, k_pool, v_pool, slots, affine) against LayerNorm (fp32) of the bf16-rounded projection pre [M, 3 H]: v its
+    bits; q and k one more bf16 rounding (2^-9 of a value), doubled for a value next to a rounding boundary."""
+    slots = torch.randperm(M + 50, device=dev, generator=g)[:M].int()
+    q = torch.full((M, H), 7.0, device=dev).bfloat16()
+    kp, vp = torch.full((M + 50, H), 7.0, device=dev).bfloat16(), torch.full((M + 50, H), 7.0, device=dev).bfloat16()
+    af = {n: torch.randn(64, device=dev, generator=g) for n in ("qn_w", "qn_b", "kn_w", "kn_b")}
+    run(q_out=q, k_pool=kp, v_pool=vp, slots=slots, H=H, **af)
+    x = pre.float().view(M, 3, H // 64, 64)
+    for got, part, n in ((q, 0, "qn"), (kp[slots.long()], 1, "kn")):
+        ref = torch.nn.functional.layer_norm(x[:, part], (64,), af[n + "_w"], af[n + "_b"], 1e-6).reshape(M, H)
+        assert bool(((got.float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()), n
+    assert torch.equal(vp[slots.long()], pre[:, 2 * H:])
+    rest = torch.ones(M + 50, dtype=torch.bool, device=dev)
+    rest[slots.long()] = False
+    assert bool((kp[rest] == 7).all()) and bool((vp[rest] == 7).all())  # no other slot is written
+
+
+@pytest.mark.parametrize("H,tiles", [(64, (0,)), (192, (0,)), (256, (0, 2, 3, 4)), (1024, (0, 2, 3, 4))])
+@pytest.mark.parametrize("stages", [1, 3, 4, 7, 16])
+def test_gemm_ring_qkv(dev, H, tiles, stages):
+    """EPI_QKV on every tile that holds whole heads."""
+    K = 64 * stages
+    for tile in tiles:
+        M = 2 * RING_SHAPE[tile][0] + 37
+        g = torch.Generator(device=dev).manual_seed(H + stages)
+        A = torch.randn(M, K, device=dev, generator=g).bfloat16()
+        W = (torch.randn(3 * H, K, device=dev, generator=g) / K ** 0.5).bfloat16()
+        bias = torch.randn(3 * H, device=dev, generator=g)
+        pre = torch.empty(M, 3 * H, device=dev).bfloat16()
+        _ring(0, 0, A, W, M, 3 * H, K, bias, pre)
+        _qkv_check(dev, lambda **kw: _ring(tile, 5, A, W, M, 3 * H, K, bias, **kw), pre, M, H, g)
+
+
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 7, 9])
+def test_gemm_ring_fp8_tiles(dev, stages):
+    """fp8 on every ring tile: equal bits between the tiles (K is summed in the same order), and against fp32 of the
+    dequantized operands bf16 out and qkv as above, GELU with MX output within e4m3's rounding (2^-4 of a value; of a
+    block's largest 1e-5 for its subnormals and 1e-3 for the fp8 MFMA's own sums)."""
+    K, H = 128 * stages, 256
+    g = torch.Generator().manual_seed(stages)
+    M = 2 * 256 + 37
+    qa, sa = of.quantize_mx(torch.randn(M, K, generator=g).bfloat16())
+    qw, sw = of.quantize_weight(torch.randn(3 * H, K, generator=g) / K ** 0.5)
+    ref = of.dequantize_mx(qa, sa).to(dev) @ of.dequantize_weight(qw, sw).to(dev).t()
+    qa, sa, qw, sw = qa.to(dev), sa.to(dev), qw.to(dev), sw.to(dev)
+    g = torch.Generator(device=dev).manual_seed(stages)
+    bias = torch.randn(3 * H, device=dev, generator=g)
+    ref = ref + bias
+    f8 = {"a_scale": sa, "a_sld": K // 32, "w_scale": sw}
+    pre, first = None, None
+    for tile in range(5):
+        out = torch.full((M, 3 * H), 7.0, device=dev).bfloat16()
+        _ring(tile, 0, qa, qw, M, 3 * H, K, bias, out, **f8)
+        assert rel(out.float(), ref) < 6e-3 and (pre is None or torch.equal(out, pre))
+        pre = out
+        codes, scales = torch.zeros(M, 3 * H, dtype=torch.uint8, device=dev), torch.zeros(M, 3 * H // 32, dtype=torch.uint8, device=dev)
+        _ring(tile, 4, qa, qw, M, 3 * H, K, bias, codes, c_scale=scales, **f8)
+        want = torch.nn.functional.gelu(ref, approximate="tanh").view(M, -1, 32)
+        got = of.dequantize_mx(codes, scales).to(dev).view(M, -1, 32)
+        assert bool(((got - want).abs() <= want.abs() / 16 + 1.1e-3 * want.abs().amax(2, keepdim=True)).all())
+        assert first is None or (torch.equal(codes, first[0]) and torch.equal(scales, first[1]))
+        first = (codes, scales)
+    for tile in (0, 2, 4):
+        _qkv_check(dev, lambda **kw: _ring(tile, 5, qa, qw, M, 3 * H, K, bias, **f8, **kw), pre, M, H, g)
+
+
+@pytest.mark.parametrize("lens,N", [([50, 50], 512), ([50, 50], 509), ([130, 1, 70], 509)], ids=str)
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_gemm_splitk_taps(dev, lens, N, epi):
+    """Taps mode with a split-K workspace (a streaming chunk's conv GEMM): rows of 16-byte multiples take the small-row
+    kernel, those of 509 columns split K."""
+    H, R, M = 512, len(lens), sum(lens)
     g = torch.Generator(device=dev).manual_seed(3)
-    R, N = len(lens), sum(lens)
-    P = torch.randn(N + 2 * R, H, device=dev, generator=g).bfloat16()
-    Wfm = (torch.randn(H, 3 * H, device=dev, generator=g) / (3 * H) ** 0.5).bfloat16()
-    bias = torch.randn(H, device=dev, generator=g)
+    P = torch.randn(M + 2 * R, H, device=dev, generator=g).bfloat16()
+    Wfm = (torch.randn(N, 3 * H, device=dev, generator=g) / (3 * H) ** 0.5).bfloat16()
+    bias, gate = torch.randn(N, device=dev, generator=g), torch.randn(N, device=dev, generator=g)
     tok_row = [r for r, t in enumerate(lens) for _ in range(t)]
     a_src = torch.tensor([i + 2 * r for i, r in enumerate(tok_row)], dtype=torch.int32, device=dev)
     full = torch.cat([P[a_src.long() + j] for j in range(3)], 1).float()
     ref = full @ Wfm.float().t() + bias
-    out = torch.zeros(N, H, device=dev)
-    _gemm(P, Wfm, bias, out, 3, a_src=a_src, lda=H, K=3 * H, ws=torch.empty(16 << 20, dtype=torch.uint8, device=dev))
-    assert rel(out, ref) < 1e-5
+    out = torch.randn(M, N, device=dev, generator=g).to({2: torch.float16, 3: torch.float32}.get(epi, torch.bfloat16))
+    ref = {1: torch.nn.functional.gelu(ref, approximate="tanh"), 2: out.float() + gate * ref}.get(epi, ref)
+    _gemm(P, Wfm, bias, out, epi, gate=gate, a_src=a_src, lda=H, K=3 * H, ws=torch.empty(16 << 20, dtype=torch.uint8, device=dev))
+    assert rel(out.float(), ref) < {0: 6e-3, 1: 6e-3, 2: 1e-3, 3: 1e-5}[epi]
 
 
 @pytest.mark.parametrize("lens,tile", [([5, 0, 1, 2, 3, 40, 0, 17, 1, 56], -1), ([400] * 3, -1), ([400] * 3, 1), ([400] * 3, 2),
