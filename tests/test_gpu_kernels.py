@@ -339,6 +339,21 @@ def test_gemm_ring_fp8_tiles(dev, stages):
         _qkv_check(dev, lambda **kw: _ring(tile, 5, qa, qw, M, 3 * H, K, bias, **f8, **kw), pre, M, H, g)
 
 
+@pytest.mark.parametrize("M", [1, 20, 129, 300])
+@pytest.mark.parametrize("N,off", [(81, 0), (80, 1), (1001, 3)])
+def test_gemm_unaligned_fp32_rows(dev, M, N, off):
+    """fp32 outputs need no alignment beyond their own 4 bytes: odd row lengths, and a first row off the 16-byte grid."""
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    A = torch.randn(M, 512, device=dev, generator=g).bfloat16()
+    W = (torch.randn(N, 512, device=dev, generator=g) / 512 ** 0.5).bfloat16()
+    bias = torch.randn(N, device=dev, generator=g)
+    buf = torch.full((M * N + off + 8,), 7.0, device=dev)
+    out = buf[off:off + M * N].view(M, N)
+    _gemm(A, W, bias, out, 3)
+    assert rel(out, A.float() @ W.float().t() + bias) < 1e-5
+    assert bool((buf[:off] == 7).all()) and bool((buf[off + M * N:] == 7).all())
+
+
 @pytest.mark.parametrize("lens,N", [([50, 50], 512), ([50, 50], 509), ([130, 1, 70], 509)], ids=str)
 @pytest.mark.parametrize("epi", [0, 1, 2, 3])
 def test_gemm_splitk_taps(dev, lens, N, epi):

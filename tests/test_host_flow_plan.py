@@ -200,3 +200,17 @@ def test_one_state_in_several_windows(enc, lasts):
         assert np.array_equal(pool.ref, want)
     enc.release(st)
     assert enc.in_use() == (0, 0, 0)
+
+
+def test_workspace_follows_the_rows():
+    """A call's workspace holds its rows' activations (under 16 KB a row of the upsampled input) and nothing of a fixed size: every
+    captured graph keeps one."""
+    L, h = _lib.lib(), _lib.P()
+    d = _lib.FlowDims(CFG.vocab, CFG.dim, CFG.heads, CFG.ffn, CFG.depth1, CFG.depth2, CFG.look, CFG.stride, CFG.mel, CFG.spk, CFG.rmax,
+                      CFG.eps_layer, CFG.eps_embed, CFG.eps_after)
+    _lib.check(L.t2w_flow_create(ctypes.byref(d), ctypes.byref(h)))
+    for R, T1 in ((1, 1), (1, 25), (16, 25)):
+        n1 = R * T1
+        need = L.t2w_flow_workspace_bytes(h, n1 + CFG.look * R, n1 + 2 * R, n1, 2 * n1 + 4 * R, 2 * n1)
+        assert 0 < need < 16384 * (2 * n1 + 4 * R) + 4096
+    L.t2w_flow_destroy(h)
