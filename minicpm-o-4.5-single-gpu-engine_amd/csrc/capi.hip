@@ -283,23 +283,19 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     }
     gq.qk = QkvOut{w.q, kp, vp, a->new_slot, k.qn_w, k.qn_b, k.kn_w, k.kn_b, d.eps_qk, H, m->g.rope_freq, a->tok_abs};
     const bool small_qkv = gemm_small_fits(gq, EPI_QKV);
-    GemmArgs gr = gq;
-    gr.qk.rfreq = nullptr;
-    const RingPlan rp_qkv = ring_plan(N, 3 * H, H, 1, true, f8);
-    if (!small_qkv && rp_qkv.cfg >= 0 && gemm_ring_fits(gr, EPI_QKV)) {
-      T2W_CHECK(gemm_ring(gr, EPI_QKV, rp_qkv.cfg, st), "qkv");
-      if (m->g.rope_freq) T2W_CHECK(rope_qk(w.q, kp, a->new_slot, a->tok_abs, m->g.rope_freq, N, H, st), "rope");
-    } else if (small_qkv || (!gemm_splits(gq) && H % 256 == 0)) {
-      // per-head q / k LayerNorm and the key / value scatter in the projection's epilogue; the small-row kernel also
-      // rotates q and k, the tile kernel leaves that to rope_qk (the sine and cosine would spill its registers)
-      if (!small_qkv) gq.qk.rfreq = nullptr;
-      T2W_CHECK(gemm_bf16(gq, EPI_QKV, st), "qkv");
-      if (!small_qkv && m->g.rope_freq) T2W_CHECK(rope_qk(w.q, kp, a->new_slot, a->tok_abs, m->g.rope_freq, N, H, st), "rope");
-    } else {
+    if (m->g.rope_freq && !small_qkv && gemm_splits(gq)) {
+      // rotary embedding of up to 1024 tokens (fewer at large widths): q and k are normalised and rotated in fp32 and
+      // rounded once, as in the small-row kernel
       T2W_CHECK(gemm_bf16(gq, EPI_BF16, st), "qkv");
       T2W_CHECK(qk_norm_scatter(w.big, k.qn_w, k.qn_b, k.kn_w, k.kn_b, d.eps_qk, w.q, kp, vp, a->new_slot, N, d.heads, st,
                                 m->g.rope_freq, a->tok_abs),
                 "qk_norm");
+    } else {
+      // per-head q / k LayerNorm and the key / value scatter in the projection's epilogue; the small-row kernel also
+      // rotates q and k, the tile kernels leave that to rope_qk (the sine and cosine would spill their registers)
+      if (!small_qkv) gq.qk.rfreq = nullptr;
+      T2W_CHECK(gemm_bf16(gq, EPI_QKV, st), "qkv");
+      if (!small_qkv && m->g.rope_freq) T2W_CHECK(rope_qk(w.q, kp, a->new_slot, a->tok_abs, m->g.rope_freq, N, H, st), "rope");
     }
     AttnArgs at;
     at.q = w.q; at.k_pool = kp; at.v_pool = vp; at.out = w.ao; at.kv_idx = a->kv_idx; at.row_start = a->row_start;

@@ -306,7 +306,7 @@ def tiny_rope():
 def test_rope_streaming(dev, tiny_rope):
     """The optional rotary embedding (none in the reference) against the oracle's: prompt setups and windows past the
     trim point, so keys cached at earlier stream positions meet queries at later ones.  Setups and two-request windows
-    (132 to 220 tokens) rotate in the split-K path's q/k kernel, one-request windows (at most 128 tokens) in the
+    (132 to 220 tokens) rotate in the q/k LayerNorm kernel after the projection, one-request windows (at most 128 tokens) in the
     small-row GEMM's epilogue.  Every call is also at least 5x further from the oracle without the embedding."""
     W, model = tiny_rope
     errs = _stream_case(W, model, graphs=False) + _stream_case(W, model, graphs=False, prompts=(60,))
@@ -314,6 +314,27 @@ def test_rope_streaming(dev, tiny_rope):
     print("rope stream rel-L2 per call", errs, "against the oracle without rope", plain)
     assert max(errs) < TOL
     assert all(p > 5 * e for p, e in zip(plain, errs))
+
+
+@pytest.mark.parametrize("others", [(40,), (100, 300), (60,) * 7])
+def test_rope_keys_rounded_once(dev, tiny_rope, others):
+    """A request's rotated keys (step 0, block 0) are the same alone (100 tokens: the small-row GEMM's epilogue) as beside
+    others (180 to 940 tokens): both normalise and rotate in fp32 and round once.  The calls sum their GEMMs in other
+    orders, which moves a bf16 rounding in a few values of a thousand; rounding before the rotation too moves a third."""
+    W, model = tiny_rope
+    g = torch.Generator().manual_seed(21)
+    mus = [torch.randn(80, t, generator=g).cuda() for t in (50, *others)]
+    spks = torch.randn(len(mus), 80, generator=g).cuda()
+    keys = []
+    for n in (1, len(mus)):
+        fd = FastDiT(model, n_slots=4096, max_streams=8)
+        caches = [fd.new_cache(keep=400) for _ in range(n)]
+        fd.solve(caches, mus[:n], spks[:n], None, [True] * n)
+        keys.append(torch.cat([fd.k_pool[0][torch.from_numpy(r.slots).long().cuda()] for r in caches[0].rows]))
+    assert keys[0].shape == (100, ROPE.hidden)
+    moved = float((keys[0] != keys[1]).float().mean())
+    print("rotated keys that differ", moved)
+    assert moved < 0.02
 
 
 def test_rope_bucketed_graphs(dev, tiny_rope):
