@@ -281,7 +281,7 @@ typedef struct {
 } t2w_ring_args;
 int t2w_gemm_ring(const t2w_ring_args* a, void* stream);
 /* t2w_gemm_bf16 with a workspace for split-K partials (256-byte aligned; up to splits x M x N fp32): a call that
- * neither the small-row kernel nor the ring tiles take (16-bit output rows that are not 16-byte aligned) and whose tile
+ * neither the small-row kernel nor the ring tiles take (output rows that are not 16-byte aligned) and whose tile
  * grid would leave most CUs idle splits K over ~512 waves and reduces the partials in a fixed order. */
 int t2w_gemm_bf16_ws(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate,
                      void* C, int ldc, int M, int N, int K, int epi, void* workspace, size_t workspace_bytes,

@@ -1,5 +1,6 @@
-// Split-K bf16 MFMA GEMM for calls with few rows whose 16-bit output rows are not 16-byte aligned, which the small-row
-// kernel, the ring tiles and the tile kernel do not take (they are two to four times faster elsewhere).
+// Split-K bf16 MFMA GEMM for calls with few rows, a workspace and output rows that are not 16-byte aligned: with 16-bit
+// outputs the small-row kernel, the ring tiles and the tile kernel do not take them (they are two to four times faster
+// elsewhere).
 //
 // Pass 1: one wave per work item (64 output columns x up to 128 rows x a slice of K).  Operand fragments go straight
 // from global memory into registers: W (the MFMA B side, columns n) and A (the A side, rows m) are read 64 contiguous

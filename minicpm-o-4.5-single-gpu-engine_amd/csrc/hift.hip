@@ -552,7 +552,7 @@ __device__ __forceinline__ float pre_fast(float v, int pre, float slope, float a
 }
 
 template <int BM>
-__global__ void __launch_bounds__(256, 2) conv_bf16_kernel(ConvDesc c, const bf16_t* __restrict__ wbf) {
+__global__ void __launch_bounds__(256, 2) conv_bf16_kernel(ConvDesc c) {
   constexpr int NWV = 4, RPP = 32;              // waves; slab rows per pass of the block (8 threads per row)
   constexpr int WTM = BM / NWV, TM = WTM / 32;  // NWV waves along time, each all 64 channels
   // loads batched across rows (slab fill, epilogue) in the 512-row tile (2 waves per SIMD, registers to spare); the
@@ -1170,8 +1170,7 @@ __global__ void __launch_bounds__(64 * CS_WAVES, 4) conv_bf16_window_kernel(Conv
   else conv_epilogue_part(c, orow, co0 + cn, ncols - cn, sum);
 }
 
-// The fp32 convolution for small grids (the f0 predictor of a streaming window: ~50 frames x 512 channels), on the
-// same plan as conv_bf16_split_kernel: 32 output rows x NB * 32 output channels per workgroup, the (tap, 32-channel input
+// The fp32 convolution for small grids (the f0 predictor of one to a few rows x 512 channels): 32 output rows x NB * 32 output channels per workgroup, the (tap, 32-channel input
 // chunk) steps split over the waves, operands straight into registers with the next step's loads in flight, fp32 MFMA
 // (v_mfma_f32_32x32x2f32; lane half h supplies channels h * 16 + u of MFMA u on both sides), blocks summed in LDS in
 // wave order.
@@ -1563,7 +1562,6 @@ __global__ void __launch_bounds__(256) snake_kernel(const float4* x, int C4, lon
   }
 }
 
-// rows 1.. of each item's ups output were written one row down; row 0 = input row 1 (ReflectionPad1d((1, 0)))
 // the mean of a stage's three ResBlock outputs, in the running sum's order: ((a + b) + c) / 3
 __global__ void __launch_bounds__(256) mean3_kernel(const float4* a, const float4* b, const float4* c, float4* y, long n4) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
@@ -1583,6 +1581,7 @@ __global__ void __launch_bounds__(256) reflect_add_kernel(const float4* x, const
   y[base + i] = make_float4(__fadd_rn(v.x, s.x), __fadd_rn(v.y, s.y), __fadd_rn(v.z, s.z), __fadd_rn(v.w, s.w));
 }
 
+// rows 1.. of each item's ups output were written one row down; row 0 = input row 1 (ReflectionPad1d((1, 0)))
 __global__ void reflect_kernel(float* x, int C, const int* off, int n_items) {
   const int it = blockIdx.y;
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1630,7 +1629,7 @@ hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st) {
     // else 64
     const long t32 = (long)cdiv(max_rows, 32) * cdiv(c.Cout, 32) * c.n_items * c.n_phase;
     const long t16 = (long)cdiv(max_rows, 16) * cdiv(c.Cout, 16) * c.n_items * c.n_phase;
-      if (t16 <= 512) {
+    if (t16 <= 512) {
       dim3 grid(cdiv(max_rows, 16), cdiv(c.Cout, 16), c.n_items * c.n_phase);
       hipLaunchKernelGGL(conv_f32_split16_kernel, grid, dim3(64 * CS_WAVES), 0, st, c);
     } else if (t32 <= 256) {
@@ -1721,7 +1720,7 @@ hipError_t conv_bf16_window(const ConvDesc* c, const int* max_rows, int n, hipSt
   return hipGetLastError();
 }
 
-hipError_t conv_bf16(const ConvDesc& c, const bf16_t* wbf, int max_rows, hipStream_t st) {
+hipError_t conv_bf16(const ConvDesc& c, int max_rows, hipStream_t st) {
   if (c.n_items <= 0 || max_rows <= 0) return hipSuccess;
   if (c.epi == EPI_SNAKE) return hipErrorInvalidValue;  // fp32 convs only
   if (c.n_phase < 1 || c.n_phase > 8 || c.s_in != 1 || c.ldx % 4 || c.ldy % 4) return hipErrorInvalidValue;
@@ -1742,12 +1741,12 @@ hipError_t conv_bf16(const ConvDesc& c, const bf16_t* wbf, int max_rows, hipStre
         hipFuncSetAttribute((const void*)conv_bf16_kernel<BM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return attr;
     dim3 grid(cdiv(max_rows, BM), cdiv(c.Cout, HB_BN), c.n_items * c.n_phase);
-    hipLaunchKernelGGL(conv_bf16_kernel<BM>, grid, dim3(256), lds, st, c, wbf);
+    hipLaunchKernelGGL(conv_bf16_kernel<BM>, grid, dim3(256), lds, st, c);
   } else {
     constexpr int BM = 128;
     const size_t lds = conv_bf16_lds(BM);
     dim3 grid(cdiv(max_rows, BM), cdiv(c.Cout, HB_BN), c.n_items * c.n_phase);
-    hipLaunchKernelGGL(conv_bf16_kernel<BM>, grid, dim3(256), lds, st, c, wbf);
+    hipLaunchKernelGGL(conv_bf16_kernel<BM>, grid, dim3(256), lds, st, c);
   }
   return hipGetLastError();
 }

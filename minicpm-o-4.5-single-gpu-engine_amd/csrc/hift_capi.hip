@@ -167,7 +167,7 @@ bool on_bf16(const Ctx& x, const ConvDesc& c) {
 int run(const Ctx& x, const ConvDesc& c, int out_cls, const char* what) {
   const int mr = x.L.mx[out_cls] / c.s_out + 2;
   if (on_bf16(x, c))
-    H_CHECK(conv_bf16(c, c.wbf, mr, x.st), what);
+    H_CHECK(conv_bf16(c, mr, x.st), what);
   else
     H_CHECK(conv_f32(c, mr, x.st), what);
   return 0;

@@ -17,7 +17,7 @@ struct ConvDesc {
   float* y; int ldy;
   const int* out_off; const int* out_len;
   const float* w; const float* bias;  // w [n_phase, Cout, taps, Cin]
-  const uint16_t* wbf;                // bf16 weights for conv_bf16 (or null)
+  const uint16_t* wbf;                // bf16 weights as the caller gave them (null: fp32 only)
   const uint16_t* wfr;                // the same weights in MFMA fragment order (conv_weight_fragments); the tile kernels read these
   int Cin, Cout, taps;
   int s_in, d_in, s_out;
@@ -29,9 +29,8 @@ struct ConvDesc {
 };
 
 hipError_t conv_f32(const ConvDesc& c, int max_rows, hipStream_t st);
-// stride-1 / polyphase convs on bf16 MFMA; wbf: bf16 weights [n_phase, Cout padded to 64, taps, Cin padded to 64], and
-// c.wfr the same weights in fragment order (the slab-tile kernels need it)
-hipError_t conv_bf16(const ConvDesc& c, const uint16_t* wbf, int max_rows, hipStream_t st);
+// stride-1 / polyphase convs on bf16 MFMA with the fragment-ordered weights c.wfr
+hipError_t conv_bf16(const ConvDesc& c, int max_rows, hipStream_t st);
 // up to CONV_BATCH independent convs of small grids (each one that fits) in one launch
 constexpr int CONV_BATCH = 3;
 // A conv is small while 128 x 64 tiles of it number fewer than this: one alone up to about one per CU, three side by

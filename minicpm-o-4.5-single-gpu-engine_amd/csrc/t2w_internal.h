@@ -13,7 +13,7 @@ typedef uint16_t f16_t;  // storage type of the fp16 residual stream
 
 // EPI_GELU_MX8: GELU, then MX fp8 codes to C (bytes, ldc) and block scales to c_scale (N % 32 == 0)
 // EPI_QKV: the attention projection (N = 3 H): q and k rounded to bf16, per-head LayerNorm + affine, q to its token
-// row of q_out, k and v to the token's key slot of the pools (fields qk.*); tile path only
+// row of q_out, k and v to the token's key slot of the pools (fields qk.*)
 // EPI_PART (small-row and ring GEMMs): K split over `splits` workgroups per tile, split z writes its fp32 sum without bias
 // to C + z * c_split (rows ldc apart); a row kernel that takes the sums as a Pend finishes the GEMM's epilogue
 // Epilogues.  EPI_RESID_F16: the gated residual C(fp16) = fp16(C + gate * (acc + bias)), the residual stream kept in the
@@ -70,9 +70,9 @@ struct Pend {
   const float* gate = nullptr;
 };
 
-// cfg < 0: by shape (split-K through g.ws when a tile grid would be too small to fill the chip)
+// cfg < 0: by shape (the small-row kernel, the ring tiles, split-K through g.ws for few rows that neither takes, tiles)
 hipError_t gemm_bf16(const GemmArgs& g, int epi, hipStream_t st, int cfg = -1);
-bool gemm_splits(const GemmArgs& g);  // whether gemm_bf16 (cfg < 0) takes the split-K path for g
+bool gemm_splits(const GemmArgs& g);  // g: few tiles and room for split-K partials
 
 // One-kernel GEMM for calls of at most GEMM_SMALL_MAX_M rows (K split over the waves of a workgroup, reduced in LDS):
 // plain epilogues (EPI_BF16 .. EPI_F32; K % 64 == 0, K <= 3072, ldc % 4 == 0), EPI_PART (the same, K also split over

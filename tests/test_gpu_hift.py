@@ -225,9 +225,9 @@ def test_workspace_holds_what_the_mode_runs(kw, mode):
     assert hm._ws.numel() == need(58, mode) and bool(torch.isfinite(out).all())
 
 
-@pytest.mark.parametrize("lens", [[1], [2, 1], [15], [16], [17, 33], [34], [35], [190], [255], [256], [257]], ids=str)
+@pytest.mark.parametrize("lens", [[1], [2, 1], [15], [16], [17, 33], [34], [35], [190], [253], [254], [255]], ids=str)
 def test_small_fp32_convs(lens):
-    """Calls of up to 256 frames run the f0 predictor's convs on 16 x 16 tiles, of up to 34 conv_post (18 channels) and of
+    """Calls of up to 254 frames (grids are sized for two rows more) run the f0 predictor's convs on 16 x 16 tiles, of up to 34 conv_post (18 channels) and of
     one or two frames most of the strict-fp32 decoder; on both sides of the tiles' edges and of the rule's.  The f0 bound
     is five fp32 convs' rounding (K = 1536 sums, relative 6e-8 x sqrt(1536) = 2.3e-6 each), the decoder's the
     reference's."""
