@@ -207,16 +207,19 @@ Defer defer_plan(const t2w_dit_dims& d, int N, int K, const Work& w, bool taps) 
   return Defer{S >= 2 && gemm_small_fits(g, EPI_PART) ? S : 1, -1};
 }
 
-// g (its bias and gate excepted) as a K-split GEMM into the partial area; the returned Pend finishes it
-Pend gemm_deferred(GemmArgs g, const Defer& df, const Work& w, hipStream_t st, hipError_t* err) {
-  Pend p;
-  p.part = w.part; p.S = df.splits; p.stride = (size_t)g.M * g.N; p.ld = g.N; p.bias = g.bias; p.gate = g.gate;
+// g (its bias and gate excepted) as a K-split GEMM into the partial area, where df plans one and its kernel takes the
+// operands (the ring copies them 16 bytes at a time: weights off that grid are not deferred); p finishes it
+bool gemm_deferred(GemmArgs g, const Defer& df, const Work& w, hipStream_t st, Pend* p, hipError_t* err) {
+  if (df.splits < 2) return false;
+  const Pend pd{w.part, df.splits, (size_t)g.M * g.N, g.N, g.bias, g.gate};
   g.C = w.part;
   g.ldc = g.N;
   g.splits = df.splits;
-  g.c_split = p.stride;
+  g.c_split = pd.stride;
+  if (df.ring_cfg >= 0 && !gemm_ring_fits(g, EPI_PART)) return false;
+  *p = pd;
   *err = df.ring_cfg < 0 ? gemm_small(g, EPI_PART, st) : gemm_ring(g, EPI_PART, df.ring_cfg, st);
-  return p;
+  return true;
 }
 
 // One estimator evaluation from w.a_in (bf16 [N, 4 mel]) to w.dphi (fp32 [N, mel]) at Euler step `step`.
@@ -283,9 +286,11 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     }
     gq.qk = QkvOut{w.q, kp, vp, a->new_slot, k.qn_w, k.qn_b, k.kn_w, k.kn_b, d.eps_qk, H, m->g.rope_freq, a->tok_abs};
     const bool small_qkv = gemm_small_fits(gq, EPI_QKV);
-    if (m->g.rope_freq && !small_qkv && gemm_splits(gq)) {
+    GemmArgs gr = gq;
+    gr.qk.rfreq = nullptr;
+    if (!small_qkv && gemm_splits(gq) && (m->g.rope_freq || !gemm_ring_fits(gr, EPI_QKV))) {
       // rotary embedding of up to 1024 tokens (fewer at large widths): q and k are normalised and rotated in fp32 and
-      // rounded once, as in the small-row kernel
+      // rounded once, as in the small-row kernel.  Or weights off the ring's 16-byte grid, which split K
       T2W_CHECK(gemm_bf16(gq, EPI_BF16, st), "qkv");
       T2W_CHECK(qk_norm_scatter(w.big, k.qn_w, k.qn_b, k.kn_w, k.kn_b, d.eps_qk, w.q, kp, vp, a->new_slot, N, d.heads, st,
                                 m->g.rope_freq, a->tok_abs),
@@ -313,20 +318,17 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
                           f8 ? k8->fc1_w8 : k.fc1_w, f8 ? k8->fc2_w8 : k.fc2_w, f8 ? m->blocks8[bn].qkv_w8 : kn.qkv_w};
       const size_t HH = eb * H * H, HF = eb * H * F, wb[] = {HH, 3 * HH, 3 * HH, HF, HF, 3 * HH};
       static_assert(sizeof(wb) / sizeof(wb[0]) == AttnArgs::PF_RANGES, "one range per weight");
-      for (int r = 0; r < AttnArgs::PF_RANGES; ++r) at.pf[r] = wp[r], at.pf_bytes[r] = wb[r];
+      for (int r = 0; r < AttnArgs::PF_RANGES; ++r) at.pf[r] = wp[r], at.pf_bytes[r] = (uintptr_t)wp[r] & 15 ? 0 : wb[r];
     }
     T2W_CHECK(attention(at, st), "attention");
     if (f8)
       T2W_CHECK(gemm_bf16(gemm8(w.o8, H, nullptr, w.o8s, k8->proj_w8, k8->proj_ws, k.proj_b, g_a, w.h, H, N, H, H), EPI_RESID_F16, st), "proj");
-    else if (df_proj.splits > 1) {
+    else {
       const void* pw = wt(k.proj_w, k8 ? k8->proj_w8 : nullptr, k8 ? k8->proj_ws : nullptr, H, H);
       T2W_CHECK(derr, "dequant proj");
-      pend = gemm_deferred(gemm_args(w.ao, H, nullptr, pw, k.proj_b, g_a, w.h, H, N, H, H, &w), df_proj, w, st, &perr);
-      T2W_CHECK(perr, "proj");
-    } else {
-      const void* pw = wt(k.proj_w, k8 ? k8->proj_w8 : nullptr, k8 ? k8->proj_ws : nullptr, H, H);
-      T2W_CHECK(derr, "dequant proj");
-      T2W_CHECK(timed_launch(T2W_TIMER_RESID_GEMM, resid_bytes(N, H, H), st, [&] { return gemm_bf16(gemm_args(w.ao, H, nullptr, pw, k.proj_b, g_a, w.h, H, N, H, H, &w), EPI_RESID_F16, st); }), "proj");
+      const GemmArgs gp = gemm_args(w.ao, H, nullptr, pw, k.proj_b, g_a, w.h, H, N, H, H, &w);
+      if (gemm_deferred(gp, df_proj, w, st, &pend, &perr)) T2W_CHECK(perr, "proj");
+      else T2W_CHECK(timed_launch(T2W_TIMER_RESID_GEMM, resid_bytes(N, H, H), st, [&] { return gemm_bf16(gp, EPI_RESID_F16, st); }), "proj");
     }
     ConvPlace cp;
     cp.P = w.P; cp.tok_row = a->tok_row; cp.tok_pos = a->tok_pos; cp.row_start = a->row_start; cp.row_len = a->row_len;
@@ -343,12 +345,9 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     } else {
       const void* cw = wt(k.c1_w, k8 ? k8->c1_w8 : nullptr, k8 ? k8->c1_ws : nullptr, H, 3 * H);
       T2W_CHECK(derr, "dequant conv1");
-      if (df_conv.splits > 1) {
-        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w), df_conv, w, st, &perr);
-        T2W_CHECK(perr, "conv1");
-      } else {
-        T2W_CHECK(gemm_bf16(gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w), EPI_BF16, st), "conv1");
-      }
+      const GemmArgs gc = gemm_args(w.P, H, a->a_src, cw, k.c1_b, nullptr, w.ao, H, N, H, 3 * H, &w);
+      if (gemm_deferred(gc, df_conv, w, st, &pend, &perr)) T2W_CHECK(perr, "conv1");
+      else T2W_CHECK(gemm_bf16(gc, EPI_BF16, st), "conv1");
     }
     cp.cache_base = cbase + 2 * H;
     cp.cache_out_base = cbase + 2 * H;
@@ -360,12 +359,9 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
     } else {
       const void* cw = wt(k.c2_w, k8 ? k8->c2_w8 : nullptr, k8 ? k8->c2_ws : nullptr, H, 3 * H);
       T2W_CHECK(derr, "dequant conv2");
-      if (df_conv.splits > 1) {
-        pend = gemm_deferred(gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w), df_conv, w, st, &perr);
-        T2W_CHECK(perr, "conv2");
-      } else {
-        T2W_CHECK(gemm_bf16(gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w), EPI_RESID_F16, st), "conv2");
-      }
+      const GemmArgs gc = gemm_args(w.P, H, a->a_src, cw, k.c2_b, g_c, w.h, H, N, H, 3 * H, &w);
+      if (gemm_deferred(gc, df_conv, w, st, &pend, &perr)) T2W_CHECK(perr, "conv2");
+      else T2W_CHECK(gemm_bf16(gc, EPI_RESID_F16, st), "conv2");
     }
     if (f8) {
       T2W_CHECK(ln_mod_mx8(w.h, sh_m, sc_m, d.eps_block, w.a8, w.a8s, N, H, st,
@@ -384,12 +380,9 @@ int run_estimator(const t2w_dit* m, const t2w_solve_args* a, const Work& w, int 
       T2W_CHECK(gemm_bf16(gemm_args(w.abuf, H, nullptr, f1w, k.fc1_b, nullptr, w.big, F, N, F, H, &w), EPI_GELU_BF16, st), "fc1");
       const void* f2w = wt(k.fc2_w, k8 ? k8->fc2_w8 : nullptr, k8 ? k8->fc2_ws : nullptr, H, F);
       T2W_CHECK(derr, "dequant fc2");
-      if (df_fc2.splits > 1) {
-        pend = gemm_deferred(gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w), df_fc2, w, st, &perr);
-        T2W_CHECK(perr, "fc2");
-      } else {
-        T2W_CHECK(timed_launch(T2W_TIMER_RESID_GEMM, resid_bytes(N, H, F), st, [&] { return gemm_bf16(gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w), EPI_RESID_F16, st); }), "fc2");
-      }
+      const GemmArgs g2 = gemm_args(w.big, F, nullptr, f2w, k.fc2_b, g_m, w.h, H, N, H, F, &w);
+      if (gemm_deferred(g2, df_fc2, w, st, &pend, &perr)) T2W_CHECK(perr, "fc2");
+      else T2W_CHECK(timed_launch(T2W_TIMER_RESID_GEMM, resid_bytes(N, H, F), st, [&] { return gemm_bf16(g2, EPI_RESID_F16, st); }), "fc2");
     }
   }
   T2W_CHECK(ln_mod(w.h, fmods, fmods + H, d.eps_final, w.abuf, N, H, st, pend), "final norm");

@@ -5,10 +5,13 @@ the fp32 oracle (the reference's own fast-vs-reference FP16 bounds are 2e-2 for 
 ``tests/engine/test_dit_fast.py:86,103`` of the reference); measured values are printed.
 """
 
+import ctypes
+
 import pytest
 import torch
 
 import t2w_amd  # noqa: F401
+from t2w_amd import _lib
 from t2w_amd.config import DiTConfig
 from t2w_amd.dit import DiTModel, FastDiT
 from t2w_amd.weights import init_dit
@@ -287,6 +290,34 @@ def test_fp8_streaming_vs_oracle(dev):
         errs.append(rel(got[0].cpu(), ref[0]))
     print("fp8 streaming vs oracle rel-L2 per window", errs)
     assert max(errs) < FP8_TOL
+
+
+@pytest.mark.parametrize("Ts", [(50,), (70, 30), (100, 150, 200)], ids=str)
+def test_weights_off_the_16_byte_grid(dev, tiny, Ts):
+    """Block weights need no more than their own alignment in calls of up to 1024 tokens (here views 8 bytes into their
+    memory; 100, 200 and 900 tokens): the mel of the aligned weights, up to the order of sums (another kernel may take
+    the GEMM; 7e-4 where every GEMM of a full-size solve changed its order, bound 4 times that)."""
+    W, model = tiny
+    off = DiTModel(W, TINY)
+    for b, blk in enumerate(off.blocks):
+        for n in ("qkv_w", "proj_w", "c1_w", "c2_w", "fc1_w", "fc2_w"):
+            buf = torch.empty(blk[n].numel() + 4, dtype=torch.bfloat16, device=dev)
+            blk[n] = buf[4:].view(blk[n].shape).copy_(blk[n])
+            assert blk[n].data_ptr() % 16 == 8
+        s = _lib.DitBlock(*[blk[n].data_ptr() for n, _ in _lib.DitBlock._fields_])
+        _lib.check(_lib.lib().t2w_dit_set_block(off.handle, b, ctypes.byref(s)), "set_block")
+    g = torch.Generator().manual_seed(23)
+    mus = [torch.randn(80, t, generator=g).cuda() for t in Ts]
+    spks = torch.randn(len(Ts), 80, generator=g).cuda()
+    want, got = [], []
+    for m, out in ((model, want), (off, got)):
+        fd = FastDiT(m, n_slots=4096, max_streams=4)
+        caches = [fd.new_cache() for _ in Ts]
+        for _ in range(2):  # the second window over the first's keys
+            out += fd.solve(caches, mus, spks, None, [True] * len(Ts))
+    errs = [rel(a, b) for a, b in zip(got, want)]
+    print("misaligned weights rel-L2", errs)
+    assert max(errs) < 3e-3
 
 
 ROPE = DiTConfig(hidden=256, depth=2, heads=4, ffn=512, rope_theta=10000.0)
