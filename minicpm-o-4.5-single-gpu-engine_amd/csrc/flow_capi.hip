@@ -35,11 +35,16 @@ int ferr(const char* what, hipError_t e = hipSuccess) { return set_error(what, e
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// K-split sums of models whose GEMMs may not fit the ring's 16-byte copies and stores (split_k); other models' run on the
+// small-row kernel, the ring tiles and the tile kernel, and have no such area
+constexpr size_t FLOW_SPLITK_BYTES = (size_t)16 << 20;
+
 struct FWork {
   bf16_t* x0; bf16_t* G; f16_t* h1; bf16_t* U; float* Y; f16_t* h2; bf16_t* A; f16_t* qkv; bf16_t* ao; bf16_t* F;
+  float* part;  // or null
 };
 
-size_t fcarve(const t2w_flow_dims& d, int n_in, int n_gap, int n1, int n_up, int n2, char* base, FWork* w) {
+size_t fcarve(const t2w_flow_dims& d, int n_in, int n_gap, int n1, int n_up, int n2, bool split_k, char* base, FWork* w) {
   const size_t C = d.dim, nm = (size_t)(n1 > n2 ? n1 : n2);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes); return base ? (void*)(base + o) : nullptr; };
@@ -54,13 +59,16 @@ size_t fcarve(const t2w_flow_dims& d, int n_in, int n_gap, int n1, int n_up, int
   t.qkv = (f16_t*)take(nm * 3 * C * 2);
   t.ao = (bf16_t*)take(nm * C * 2);
   t.F = (bf16_t*)take(nm * (size_t)d.ffn * 2);
+  t.part = split_k ? (float*)take(FLOW_SPLITK_BYTES) : nullptr;
   if (w) *w = t;
   return off;
 }
 
 GemmArgs fgemm(const void* A, int lda, const int* a_src, const void* W, const float* bias, const float* gate, void* C, int ldc,
-               int M, int N, int K, int act = ACT_NONE) {
+               int M, int N, int K, const FWork& w, int act = ACT_NONE) {
   GemmArgs g{};
+  g.ws = w.part;
+  g.ws_bytes = w.part ? FLOW_SPLITK_BYTES : 0;
   g.A = (const bf16_t*)A;
   g.lda = lda;
   g.a_src = a_src;
@@ -84,8 +92,13 @@ struct t2w_flow {
   t2w_flow_dims d;
   std::vector<t2w_flow_layer> layers;
   std::vector<bool> layer_set;
-  t2w_flow_globals g;
+  t2w_flow_globals g{};
   bool globals_set = false;
+  bool split_k() const {
+    uintptr_t bits = (uintptr_t)g.conv1_w | (uintptr_t)g.conv2_w | (uintptr_t)g.up_w | (uintptr_t)g.proj_w;
+    for (const t2w_flow_layer& k : layers) bits |= (uintptr_t)k.qkv_w | (uintptr_t)k.out_w | (uintptr_t)k.w1 | (uintptr_t)k.w2;
+    return (bits & 15) || d.mel % 4;
+  }
 };
 
 int t2w_flow_create(const t2w_flow_dims* dims, t2w_flow** out) {
@@ -122,7 +135,7 @@ void t2w_flow_destroy(t2w_flow* m) { delete m; }
 
 size_t t2w_flow_workspace_bytes(const t2w_flow* m, int n_in, int n_gap, int n1, int n_up, int n2) {
   if (!m) return 0;
-  return fcarve(m->d, n_in, n_gap, n1, n_up, n2, nullptr, nullptr);
+  return fcarve(m->d, n_in, n_gap, n1, n_up, n2, m->split_k(), nullptr, nullptr);
 }
 
 namespace {
@@ -142,7 +155,7 @@ int run_layer(const t2w_flow* m, const t2w_flow_layer& k, f16_t* h, int n, bool 
   const t2w_flow_dims& d = m->d;
   const int C = d.dim;
   if (!normed) T2W_FCHECK(ln_mod(h, k.ln1_b, k.ln1_w, d.eps_layer, w.A, n, C, st), "flow norm_mha");
-  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, k.qkv_w, k.qkv_b, nullptr, w.qkv, 3 * C, n, 3 * C, C), EPI_F16, st), "flow qkv");
+  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, k.qkv_w, k.qkv_b, nullptr, w.qkv, 3 * C, n, 3 * C, C, w), EPI_F16, st), "flow qkv");
   T2W_FCHECK(flow_kv_store(w.qkv, 3 * C, pool, new_slot, n, C, st), "flow key/value store");
   RelAttnArgs a{};
   a.qkv = w.qkv;
@@ -163,10 +176,10 @@ int run_layer(const t2w_flow* m, const t2w_flow_layer& k, f16_t* h, int n, bool 
   a.heads = d.heads;
   a.scale = 1.0f / sqrtf(64.0f);
   T2W_FCHECK(flow_rel_attention(a, st), "flow attention");
-  T2W_FCHECK(gemm_bf16(fgemm(w.ao, C, nullptr, k.out_w, k.out_b, m->g.ones, h, C, n, C, C), EPI_RESID_F16, st), "flow linear_out");
+  T2W_FCHECK(gemm_bf16(fgemm(w.ao, C, nullptr, k.out_w, k.out_b, m->g.ones, h, C, n, C, C, w), EPI_RESID_F16, st), "flow linear_out");
   T2W_FCHECK(ln_mod(h, k.ln2_b, k.ln2_w, d.eps_layer, w.A, n, C, st), "flow norm_ff");
-  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, k.w1, k.b1, nullptr, w.F, d.ffn, n, d.ffn, C, ACT_SILU), EPI_BF16, st), "flow w_1");
-  T2W_FCHECK(gemm_bf16(fgemm(w.F, d.ffn, nullptr, k.w2, k.b2, m->g.ones, h, C, n, C, d.ffn), EPI_RESID_F16, st), "flow w_2");
+  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, k.w1, k.b1, nullptr, w.F, d.ffn, n, d.ffn, C, w, ACT_SILU), EPI_BF16, st), "flow w_1");
+  T2W_FCHECK(gemm_bf16(fgemm(w.F, d.ffn, nullptr, k.w2, k.b2, m->g.ones, h, C, n, C, d.ffn, w), EPI_RESID_F16, st), "flow w_2");
   return 0;
 }
 
@@ -188,7 +201,7 @@ int t2w_flow_encode(const t2w_flow* m, const t2w_flow_args* a, void* stream) {
     return ferr("flow encoder: null argument pointer");
   if (!a->workspace || ((uintptr_t)a->workspace & 255)) return ferr("flow encoder: workspace missing or not 256-byte aligned");
   FWork w;
-  const size_t need = fcarve(d, a->n_in, a->n_gap, a->n1, a->n_up, a->n2, (char*)a->workspace, &w);
+  const size_t need = fcarve(d, a->n_in, a->n_gap, a->n1, a->n_up, a->n2, m->split_k(), (char*)a->workspace, &w);
   if (a->workspace_bytes < need) return ferr("flow encoder: workspace too small");
   const hipStream_t st = (hipStream_t)stream;
   const float xscale = sqrtf((float)C);
@@ -199,10 +212,10 @@ int t2w_flow_encode(const t2w_flow* m, const t2w_flow_args* a, void* stream) {
   T2W_FCHECK(flow_embed(g.embed_table, a->tok, a->res, g.embed_ln_w, g.embed_ln_b, d.eps_embed, xscale, w.x0, w.h1, a->n_in, C, st),
              "flow embed");
   // pre-lookahead layer: conv1 over each frame and its lookahead (leaky ReLU), its cached frames, conv2 + residual
-  T2W_FCHECK(gemm_bf16(fgemm(w.x0, C, a->c1_src, g.conv1_w, g.conv1_b, nullptr, w.G, C, a->n_gap, C, (d.look + 1) * C, ACT_LRELU),
+  T2W_FCHECK(gemm_bf16(fgemm(w.x0, C, a->c1_src, g.conv1_w, g.conv1_b, nullptr, w.G, C, a->n_gap, C, (d.look + 1) * C, w, ACT_LRELU),
                        EPI_BF16, st), "flow pre-lookahead conv1");
   T2W_FCHECK(flow_look_place(w.G, cnn, a->gofs, a->t1, a->cnn_rd, a->cnn_wr, R, C, cstride, st), "flow pre-lookahead cache");
-  T2W_FCHECK(gemm_bf16(fgemm(w.G, C, a->c2_src, g.conv2_w, g.conv2_b, g.ones, w.h1, C, a->n1, C, 3 * C), EPI_RESID_F16, st),
+  T2W_FCHECK(gemm_bf16(fgemm(w.G, C, a->c2_src, g.conv2_w, g.conv2_b, g.ones, w.h1, C, a->n1, C, 3 * C, w), EPI_RESID_F16, st),
              "flow pre-lookahead conv2");
   f16_t* pool1 = (f16_t*)a->pool1;
   for (int l = 0; l < d.depth1; ++l)
@@ -213,7 +226,7 @@ int t2w_flow_encode(const t2w_flow* m, const t2w_flow_args* a, void* stream) {
   // x sqrt(C), and the first up layer's norm
   T2W_FCHECK(flow_up_place(w.h1, w.U, a->up_dst, a->n1, a->uofs, a->o1, a->t1, cnn, a->cnn_rd, a->cnn_wr, R, C, cstride, st),
              "flow upsample frames");
-  T2W_FCHECK(gemm_bf16(fgemm(w.U, C, a->up_src, g.up_w, g.up_b, nullptr, w.Y, C, a->n2, C, (2 * d.stride + 1) * C), EPI_F32, st),
+  T2W_FCHECK(gemm_bf16(fgemm(w.U, C, a->up_src, g.up_w, g.up_b, nullptr, w.Y, C, a->n2, C, (2 * d.stride + 1) * C, w), EPI_F32, st),
              "flow upsample conv");
   const t2w_flow_layer& u0 = m->layers[d.depth1];
   T2W_FCHECK(flow_ln_scale_ln(w.Y, g.up_ln_w, g.up_ln_b, d.eps_embed, xscale, w.h2, u0.ln1_w, u0.ln1_b, d.eps_layer, w.A, a->n2, C, st),
@@ -224,7 +237,7 @@ int t2w_flow_encode(const t2w_flow* m, const t2w_flow_args* a, void* stream) {
                   a->kv2_off, a->kv2_len, a->o2, a->t2, a->tiles2, a->n_tiles2, w, st))
       return 1;
   T2W_FCHECK(ln_mod(w.h2, g.after_b, g.after_w, d.eps_after, w.A, a->n2, C, st), "flow after_norm");
-  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, g.proj_w, g.proj_b, nullptr, a->mu_out, d.mel, a->n2, d.mel, C), EPI_F32, st),
+  T2W_FCHECK(gemm_bf16(fgemm(w.A, C, nullptr, g.proj_w, g.proj_b, nullptr, a->mu_out, d.mel, a->n2, d.mel, C, w), EPI_F32, st),
              "flow encoder_proj");
   return 0;
 }

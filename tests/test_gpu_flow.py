@@ -6,6 +6,8 @@ Tolerance: bf16 MFMA GEMM inputs and fp16 keys / values / residual stream (the r
 fp32: rel-L2 of each window's ``mu`` <= 6e-3 (measured 3.4e-3 .. 3.8e-3).
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -13,6 +15,7 @@ import torch
 from oracle import flow as of
 
 import t2w_amd  # noqa: F401
+from t2w_amd import _lib
 from t2w_amd.config import FlowConfig
 from t2w_amd.flow import FlowEncoder, FlowModel
 from t2w_amd.weights import init_flow
@@ -163,3 +166,29 @@ def test_key_groups_match_oracle(flow, n):
         assert rel(mu[rows[i]:rows[i] + frames[i]].t().cpu(), refs[i % 2]) < TOL
     for st in states:
         enc.release(st)
+
+
+def test_weights_off_the_16_byte_grid(flow, dev):
+    """GEMM weights 8 bytes into their memory: one window and a call of 280 rows (more than the small-row kernel takes),
+    against the oracle."""
+    W, d, _ = flow
+    model = FlowModel(W, FlowConfig(), device=dev)
+    off8 = lambda t: torch.empty(t.numel() + 4, dtype=t.dtype, device=dev)[4:].view(t.shape).copy_(t)  # noqa: E731
+    L = _lib.lib()
+    for n in ("conv1_w", "conv2_w", "up_w", "proj_w"):
+        model.g[n] = off8(model.g[n])
+    _lib.check(L.t2w_flow_set_globals(model.handle, ctypes.byref(_lib.FlowGlobals(**{k: v.data_ptr() for k, v in model.g.items()}))), "globals")
+    for i, lw in enumerate(model.layers):
+        for n in ("qkv_w", "out_w", "w1", "w2"):
+            lw[n] = off8(lw[n])
+            assert lw[n].data_ptr() % 16 == 8
+        _lib.check(L.t2w_flow_set_layer(model.handle, i, ctypes.byref(_lib.FlowLayer(**{k: v.data_ptr() for k, v in lw.items()}))), "layer")
+    enc = FlowEncoder(model, n_slots1=4096, n_slots2=8192, n_cnn=64)
+    g = torch.Generator().manual_seed(9)
+    for lens in ((17,), (97, 43)):
+        toks = [torch.randint(0, d.vocab, (t,), generator=g).tolist() for t in lens]
+        states, mu, rows, frames = enc.setup(toks)
+        for i, p in enumerate(toks):
+            assert rel(mu[rows[i]:rows[i] + frames[i]].t().cpu(), of.setup(W, d, p)[0]) < TOL
+        for st in states:
+            enc.release(st)
