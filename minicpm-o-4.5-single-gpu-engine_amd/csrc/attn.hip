@@ -583,7 +583,9 @@ hipError_t attention(const AttnArgs& a, hipStream_t st) {
   // a grid of fewer workgroups than CUs (a streaming chunk) splits each workgroup's key tiles over four wave groups; one
   // of up to about two per CU (several streaming windows, prompts) over two, since their serial key tiles and not
   // the CUs bound it: in a solve of five windows 20.6 -> 19.1 ms, of a 300-frame prompt 20.7 -> 20.3 ms (four groups
-  // there: 19.6 and 21.4 ms; two groups on sixteen windows, 992 workgroups: no change)
+  // there: 19.6 and 21.4 ms; two groups on sixteen windows, 992 workgroups: no change).  Both counts include a bucketed
+  // call's empty tiles, and the reading workgroups hold their kernel's LDS (128 KB with four groups, 64 KB with two), so
+  // these figures are of those two things together
   if (wgs < 256) {
     hipLaunchKernelGGL(attn_kernel<4>, dim3(wgs + pfw), dim3(512), 0, st, a);
   } else if (wgs < 600) {
