@@ -155,8 +155,9 @@ int t2w_dit_solve_noalloc(const t2w_dit* m, const t2w_solve_args* a, void* strea
  * thread; the eager (not capturing) calls that follow bracket each instrumented kernel launch with a pair of HIP events
  * on its stream, up to cap launches.  t2w_timer_read waits for `stream`, writes the launches' kinds, durations (ms)
  * and algorithmic HBM bytes (the least its operands make it move) in launch order, up to cap, their count to *n,
- * and disarms.  Instrumented: the DiT's dense gated-residual tile GEMMs (proj and fc2 of every block, calls of more
- * than 128 tokens) and HiFT's elementwise kernels. */
+ * and disarms.  Instrumented: the DiT's dense gated-residual GEMMs (proj and fc2 of every block, calls of more than
+ * 128 tokens; where K is split over workgroups, the launch that leaves the sums to the next row kernel) and HiFT's
+ * elementwise kernels. */
 enum {
   T2W_TIMER_RESID_GEMM = 1,
   T2W_TIMER_HIFT_PHASE = 2,

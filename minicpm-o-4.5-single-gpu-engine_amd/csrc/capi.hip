@@ -208,7 +208,8 @@ Defer defer_plan(const t2w_dit_dims& d, int N, int K, const Work& w, bool taps) 
 }
 
 // g (its bias and gate excepted) as a K-split GEMM into the partial area, where df plans one and its kernel takes the
-// operands (the ring copies them 16 bytes at a time: weights off that grid are not deferred); p finishes it
+// operands (the ring copies them 16 bytes at a time: weights off that grid are not deferred); p finishes it.  Gated
+// residuals of more than GEMM_SMALL_MAX_M dense rows are timed as such, with the bytes of this launch: operands and sums
 bool gemm_deferred(GemmArgs g, const Defer& df, const Work& w, hipStream_t st, Pend* p, hipError_t* err) {
   if (df.splits < 2) return false;
   const Pend pd{w.part, df.splits, (size_t)g.M * g.N, g.N, g.bias, g.gate};
@@ -218,7 +219,10 @@ bool gemm_deferred(GemmArgs g, const Defer& df, const Work& w, hipStream_t st, P
   g.c_split = pd.stride;
   if (df.ring_cfg >= 0 && !gemm_ring_fits(g, EPI_PART)) return false;
   *p = pd;
-  *err = df.ring_cfg < 0 ? gemm_small(g, EPI_PART, st) : gemm_ring(g, EPI_PART, df.ring_cfg, st);
+  auto launch = [&] { return df.ring_cfg < 0 ? gemm_small(g, EPI_PART, st) : gemm_ring(g, EPI_PART, df.ring_cfg, st); };
+  const double M = g.M, N = g.N, K = g.K;
+  *err = pd.gate && !g.a_src && g.M > GEMM_SMALL_MAX_M
+             ? timed_launch(T2W_TIMER_RESID_GEMM, 2 * M * K + 2 * N * K + 4 * M * N * g.splits, st, launch) : launch();
   return true;
 }
 

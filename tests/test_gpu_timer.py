@@ -38,6 +38,24 @@ def test_solve_timed_counts_and_bits(dev):
     print("timed proj/fc2 launches", len(launches), "mean ms", sum(m for _, m, _ in launches) / len(launches))
 
 
+@pytest.mark.parametrize("T", [65, 150, 512])
+def test_mid_size_solve_timed(dev, T):
+    """Calls of 129 to 1024 tokens (here 130, 300 and 1024) time their proj and fc2 launches too, whether K is split or
+    not; the mel is the untimed solve's."""
+    model = DiTModel(init_dit(TINY, seed=12), TINY)
+    g = torch.Generator().manual_seed(2)
+    mu, spk = torch.randn(80, T, generator=g).cuda(), torch.randn(1, 80, generator=g).cuda()
+    outs = []
+    for timed in (False, True):
+        fd = FastDiT(model, n_slots=4096, max_streams=2)
+        args = ([fd.new_cache()], [mu], spk, None, [False])
+        mels, launches = fd.solve_timed(*args) if timed else (fd.solve(*args), [])
+        outs.append(mels[0])
+    assert torch.equal(outs[0], outs[1])
+    assert [k for k, _, _ in launches] == ["resid_gemm"] * (2 * TINY.depth * TINY.steps)
+    assert all(ms > 0 and by > 0 for _, ms, by in launches)
+
+
 def test_hift_stages_timed_and_graphs_untimed(dev):
     """HiFT's elementwise stages are timed in an eager call (strict fp32: Snake too); a graph replay records nothing."""
     W = init_hift(HiFTConfig(), seed=5)
